@@ -4,30 +4,29 @@
 // Replaces the nn.Linear projections of a recurrent step as the reference runs
 // them through torch (q/k/v/o_proj ouro/modeling_ouro.py:371-374,390-392,431;
 // gate/up/down_proj :162-168; Huginn Wqkv/proj/fc/adapter
-// huginn/modeling_huginn.py:239-242,310-316,372). With at most 64 rows the
-// product is bound by streaming W from HBM (2 flops per weight element per
-// row, far under the MFMA ridge), so the kernel is built to keep that stream
-// deep rather than to reuse tiles:
+// huginn/modeling_huginn.py:239-242,310-316,372). The product is bound by
+// streaming W from HBM (2 flops per weight element per row, under the MFMA
+// ridge up to a few hundred rows), so every form is built to keep that stream
+// deep. Three forms share one packed weight: the row kernel (few rows, K split
+// over a workgroup's waves; also the LM head's argmax), a split-K form for few
+// rows, and the streaming form for the rest.
 //   * W is stored pre-packed in MFMA operand order (cdb_linear_pack_weight):
 //     for each tile of 16 rows and each 32-element contraction step, the 1 KiB
 //     block that one wave loads as its A operand -- lane (r, g) holding
 //     W[16 t + r][32 s + 8 g .. +8] -- is contiguous, and a tile's blocks follow
 //     each other along K. Every weight load is one fully contiguous 1 KiB wave
 //     access, and a wave's batch of S steps is S KiB in a row;
-//   * a workgroup owns NB tiles of 16 output columns and splits the contraction
-//     dimension K between its waves; every weight element is read exactly once,
-//     with non-temporal loads so x stays resident in L2;
-//   * MFMA 16x16x32 bf16 with A = 16 rows of W and B = x^T (up to 4 tiles of
-//     16 rows of x): lane (m, g) loads x[m][32 s + 8 g .. +8], the same
-//     contraction indices as its A vector, and the accumulator C[n][m] lands
-//     in lane (m % 16, n / 4);
-//   * the waves' partial tiles are summed in LDS in a fixed order (slot w holds
-//     wave w + wave w+8), so results do not depend on scheduling;
-//   * gated mode (the MLP's gate_up): the workgroup also owns the matching 16
+//   * weight loads are non-temporal, so x stays resident in L2;
+//   * MFMA 16x16x32 bf16 with A = 16 rows of W and B = x^T: lane (m, g) holds
+//     x[m][32 s + 8 g .. +8], the same contraction indices as its A vector, and
+//     the accumulator C[n][m] lands in lane (m % 16, n / 4);
+//   * gated mode (the MLP's gate_up): a wave also owns the matching 16
 //     up-projection rows W[N + n] and writes R(R(silu(R(g))) * R(u)) directly,
 //     the rounding chain of torch's bf16 silu and multiply, so the [rows, 2N]
 //     gate_up activation never reaches memory.
 // Output rows are rounded to bf16 once, after the fp32 sum over all of K.
+
+#include <type_traits>
 
 #include "cdb_common.h"
 #include "../../include/cdb_amd.h"
@@ -82,16 +81,19 @@ CDB_DEVICE f32x4_t sum_slots(const f32x4_t (&red)[SLOTS][NT][MT][kWave], int til
   return v;
 }
 
+// The row kernel. A workgroup owns NB tiles of 16 output columns and splits the
+// contraction dimension K between its waves, whose partial tiles are summed in LDS
+// in a fixed order, so results do not depend on scheduling.
 // MT: 16-row tiles of x (1, 2 or 4). NB: 16-column tiles of y per workgroup; every
-// wave computes all of them, so each x vector it loads feeds NB (gated: 2*NB)
+// wave computes all of them, so each x vector it loads feeds NB
 // MFMAs. S: contraction steps loaded per batch. SLOTS: LDS partial tiles (waves
 // w, w + SLOTS, w + 2*SLOTS, ... add into slot w in that order). ARGMAX: instead
 // of y, store each row's greedy-argmax candidate of every 16-column tile (the
 // largest bf16-rounded output and its first column, torch.argmax order), for
 // linear_argmax_merge_kernel.
-template <int MT, int NB, int S, int SLOTS, bool GATED, int MAXT, bool ARGMAX = false>
+template <int MT, int NB, int S, int SLOTS, int MAXT, bool ARGMAX = false>
 __global__ void __launch_bounds__(MAXT) linear_kernel(LinearParams p) {
-  constexpr int NT = GATED ? 2 * NB : NB;  // W row tiles: gate tiles, then up tiles
+  constexpr int NT = NB;
   __shared__ f32x4_t red[SLOTS][NT][MT][kWave];
 
   const int lane = threadIdx.x & (kWave - 1);
@@ -105,10 +107,7 @@ __global__ void __launch_bounds__(MAXT) linear_kernel(LinearParams p) {
   const int total = p.K / 32;
   const bf16_t* wrow[NT];
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
-    wrow[j] = p.w + ((int64_t)(n0 / 16 + j) * total) * 512 + 8 * lane;
-    if constexpr (GATED) wrow[NB + j] = p.w + ((int64_t)((p.N + n0) / 16 + j) * total) * 512 + 8 * lane;
-  }
+  for (int j = 0; j < NB; ++j) wrow[j] = p.w + ((int64_t)(n0 / 16 + j) * total) * 512 + 8 * lane;
   const bf16_t* xrow[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) xrow[mt] = p.x + (int64_t)min(mt * 16 + r, p.M - 1) * p.ldx + 8 * g;
@@ -213,104 +212,70 @@ __global__ void __launch_bounds__(MAXT) linear_kernel(LinearParams p) {
     const int m = mt * 16 + (l & 15);
     if (m < p.M) {
       const f32x4_t v = sum_slots(red, j, mt, l, slots);
-      f32x4_t u = {};
-      if constexpr (GATED) u = sum_slots(red, NB + j, mt, l, slots);
       Vec<bf16_t, 4> o;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if constexpr (GATED) {
-          const float gate = round_bf16(v[i]);
-          const float act = silu_bf16(gate);
-          o.set(i, act * round_bf16(u[i]));
-        } else {
-          o.set(i, v[i]);
-        }
-      }
+      for (int i = 0; i < 4; ++i) o.set(i, v[i]);
       o.store(p.y + (int64_t)m * p.ldy + n0 + 16 * j + 4 * (l >> 4));
     }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Wide-tile variant for batches of 33 to 256 rows. A workgroup owns 16*MT rows
-// x 4*16*NTW columns with the full K; wave w owns column tiles w*NTW .. and
-// every row tile, so each weight byte is loaded by exactly one wave:
-//   * weight blocks stream from the packed layout into a ring of STAGES chunks
-//     of registers (SC steps each), STAGES chunks ahead of the MFMAs that use
-//     them, so the HBM latency is covered without waiting per chunk;
-//   * x chunks go through LDS, double-buffered, in operand order (16-byte
-//     unit (r, g) of block (row tile, step) holds x[16 t + r][32 s + 8 g ..]);
-//   * workgroups of one column range (different row ranges) sit on one XCD,
-//     so the weights cross HBM once;
-//   * PIPE: x chunks are triple-buffered and stored two chunks ahead, and each
-//     step's x operands are read from LDS while the previous step's MFMAs run
-//     (without it a step's reads wait for the previous step's last MFMA, and
-//     its MFMAs for the reads). Every output still adds its K steps in order
-//     in one accumulator, so the results are bit-identical either way.
+// Split-K form for few rows. A workgroup covers 16*MT rows x 64 columns of one of
+// KSPLIT K ranges and stores fp32 partial sums to p.parts[range], for a consumer
+// that adds them in range order and rounds once (the residual RMSNorm). Wave w
+// owns column tile w; weight blocks stream into a ring of kPartsStages chunks of
+// registers, and x goes through LDS, double-buffered, in operand order. A range
+// is only 16 to 70 steps: the ring holds 16 of them, loaded before anything is
+// waited for, and the chunk loop unrolls completely, so the launch is close to
+// one memory round trip. The streaming form below, whose first product waits for
+// its producer's first chunk, is slower here (us, cold weights): 5632 -> 2048 at
+// 1 / 16 / 48 / 64 rows 5.7 / 5.8 / 7.4 / 7.8 against 6.4 / 6.6 / 7.7 / 8.4;
+// 2048 -> 2048 at 1 row 3.9 against 4.1; 5280 -> 5280 at 1 / 16 rows 10.8 / 11.2
+// against 11.6 / 12.1. Above those rows it is the faster one (see dispatch_parts).
 // ---------------------------------------------------------------------------
+constexpr int kPartsStages = 4;
+constexpr int kPartsSteps = 4;  // steps per chunk
+
 // Slot of x unit (row r of a 16-row tile, step t of the chunk, k group g) within
 // its 64-unit block: the MFMA lane that reads it is r + 16 g, with r swizzled by
-// an XOR of (t, g) so that the eight (SC = 2) or sixteen (SC = 4) units one row
-// contributes to a chunk -- stored by consecutive threads -- land on distinct
-// LDS banks. For each (t, g) the XOR permutes r, so a step's 64 units stay one
-// contiguous block and the reads stay conflict-free.
-template <int SC>
-CDB_DEVICE int x_slot(int r, int t, int g) {
-  static_assert(SC == 2 || SC == 4, "x chunks of 2 or 4 steps");
-  const int sw = SC == 2 ? 2 * (4 * (t & 1) + g) : 4 * (t & 3) + g;
-  return (r ^ sw) + 16 * g;
-}
+// an XOR of (t, g) so that the sixteen units one row contributes to a chunk --
+// stored by consecutive threads -- land on distinct LDS banks. For each (t, g) the
+// XOR permutes r, so a step's 64 units stay one contiguous block and the reads
+// stay conflict-free.
+CDB_DEVICE int x_slot(int r, int t, int g) { return (r ^ (4 * (t & 3) + g)) + 16 * g; }
 
-// KSPLIT > 1: K is cut into KSPLIT ranges of KSTEPS steps; each workgroup covers
-// one range and stores fp32 partial sums to p.parts[split], for a consumer that
-// adds them in split order and rounds once (the residual RMSNorm).
-// NTAIL: N is a multiple of 16 but not of 64 * NTW, so the last column range is
-// narrower; without it N must be a multiple of 64 * NTW.
-template <int MT, int NTW, int SC, int STAGES, bool GATED, int KSTEPS, int KSPLIT = 1, bool NTAIL = false,
-          bool PIPE = false>
-__global__ void __launch_bounds__(256) linear_wide_kernel(LinearParams p) {
-  constexpr int NT = GATED ? 2 * NTW : NTW;
+// NTAIL: N is a multiple of 16 but not of 64, so the last column range is narrower;
+// without it N must be a multiple of 64.
+template <int MT, int KSTEPS, int KSPLIT, bool NTAIL>
+__global__ void __launch_bounds__(256) linear_parts_kernel(LinearParams p) {
+  constexpr int SC = kPartsSteps, STAGES = kPartsStages;
   constexpr int ROWS = 16 * MT;
   constexpr int KC = 32 * SC;
-  constexpr int UNITS = ROWS * KC / 8;
-  static_assert(UNITS % 256 == 0, "x chunk must split evenly over the workgroup");
-  static_assert(!PIPE || STAGES >= 3, "the pipelined form stores x two chunks ahead of its use");
-  constexpr int UPT = UNITS / 256;
-  __shared__ bf16x8_t xs[PIPE ? 3 : 2][MT][SC][kWave];
+  constexpr int UPT = ROWS * KC / 8 / 256;  // x units per thread and chunk
+  __shared__ bf16x8_t xs[2][MT][SC][kWave];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
 
-  // Workgroups that share a (column range, K split) -- all its row ranges -- sit on one XCD.
-  // With NTAIL the last column range may cover fewer than 4 * NTW 16-column tiles, and
+  // Workgroups that share a (column range, K range) -- all its row ranges -- sit on one XCD.
+  // With NTAIL the last column range may cover fewer than four 16-column tiles, and
   // the waves past N load the last tile (in bounds) and store nothing.
-  const int n_tiles = NTAIL ? (p.N / 16 + 4 * NTW - 1) / (4 * NTW) : p.N / (64 * NTW);
+  const int n_tiles = NTAIL ? (p.N / 16 + 3) / 4 : p.N / 64;
   const int m_tiles = (p.M + ROWS - 1) / ROWS;
   const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
-  const int mi = q % m_tiles;
-  const int pair = (q / m_tiles) * 8 + xcd;  // column range + K split
+  const int pair = (q / m_tiles) * 8 + xcd;  // column range + K range
   if (pair >= n_tiles * KSPLIT) return;     // padding workgroup of the XCD-major order: exits before any barrier
   const int ni = pair % n_tiles, ks = pair / n_tiles;
-  const int m0 = mi * ROWS;
-  const int n0 = ni * 64 * NTW;
+  const int m0 = (q % m_tiles) * ROWS;
+  const int n0 = ni * 64;
 
-  // The K range is a compile-time constant so the chunk loop unrolls completely:
-  // the compiler's wait-count pass then sees every load of the register rings in
-  // order and waits exactly for the chunk it is about to use.
-  constexpr int total = KSTEPS;
-  constexpr int nchunks = (total + SC - 1) / SC;
+  constexpr int nchunks = (KSTEPS + SC - 1) / SC;
   const int tile_steps = p.K / 32;  // steps of one packed weight tile
   const int k_first = ks * KSTEPS;
-  const bf16_t* wp[NT];
-#pragma unroll
-  for (int j = 0; j < NTW; ++j) {
-    const int tile = NTAIL ? min(n0 / 16 + wave * NTW + j, p.N / 16 - 1) : n0 / 16 + wave * NTW + j;
-    wp[j] = p.w + ((int64_t)tile * tile_steps + k_first) * 512 + 8 * lane;
-    if constexpr (GATED)
-      wp[NTW + j] = p.w + ((int64_t)(NTAIL ? p.N / 16 + tile : (p.N + n0) / 16 + wave * NTW + j) * tile_steps +
-                           k_first) * 512 + 8 * lane;
-  }
+  const int tile = NTAIL ? min(n0 / 16 + wave, p.N / 16 - 1) : n0 / 16 + wave;
+  const bf16_t* wp = p.w + ((int64_t)tile * tile_steps + k_first) * 512 + 8 * lane;
   // x staging: thread unit u reads 16 bytes of one row (units of a row are
   // consecutive, so the global reads coalesce) and stores them to that row's
   // operand slot in LDS.
@@ -322,39 +287,33 @@ __global__ void __launch_bounds__(256) linear_wide_kernel(LinearParams p) {
     const int row = u / (KC / 8), k8 = u % (KC / 8);
     xsrc[i] = p.x + (int64_t)min(m0 + row, p.M - 1) * p.ldx + (int64_t)k_first * 32;
     xk[i] = 8 * k8;
-    xdst[i] = (((row >> 4) * SC + (k8 >> 2)) * kWave) + x_slot<SC>(row & 15, k8 >> 2, k8 & 3);
+    xdst[i] = (((row >> 4) * SC + (k8 >> 2)) * kWave) + x_slot(row & 15, k8 >> 2, k8 & 3);
   }
   // This lane's operand unit (row lane % 16, k group lane / 16) of each step.
   int xrd[SC];
 #pragma unroll
-  for (int t = 0; t < SC; ++t) xrd[t] = x_slot<SC>(lane & 15, t, lane >> 4);
+  for (int t = 0; t < SC; ++t) xrd[t] = x_slot(lane & 15, t, lane >> 4);
   auto load_x = [&](int c, bf16x8_t (&xr)[UPT]) {
 #pragma unroll
-    for (int i = 0; i < UPT; ++i) xr[i] = cdb::load_x(xsrc[i] + min(c * KC + xk[i], total * 32 - 8));
+    for (int i = 0; i < UPT; ++i) xr[i] = cdb::load_x(xsrc[i] + min(c * KC + xk[i], KSTEPS * 32 - 8));
   };
   auto store_x = [&](int buf, const bf16x8_t (&xr)[UPT]) {
     bf16x8_t* base = &xs[buf][0][0][0];
 #pragma unroll
     for (int i = 0; i < UPT; ++i) base[xdst[i]] = xr[i];
   };
-  auto load_w = [&](int c, bf16x8_t (&wr)[NT][SC]) {
+  auto load_w = [&](int c, bf16x8_t (&wr)[SC]) {
 #pragma unroll
-    for (int t = 0; t < SC; ++t) {
-      const int64_t blk = (int64_t)min(c * SC + t, total - 1) * 512;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) wr[nt][t] = cdb::load_w(wp[nt] + blk);
-    }
+    for (int t = 0; t < SC; ++t) wr[t] = cdb::load_w(wp + (int64_t)min(c * SC + t, KSTEPS - 1) * 512);
   };
 
-  f32x4_t acc[NT][MT];
+  f32x4_t acc[MT];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   // Chunk j's weights live in ring[j % STAGES] and its x in xring[j % STAGES] from STAGES
-  // chunks before it is used; x moves to LDS one chunk ahead of its MFMAs (two with PIPE).
-  bf16x8_t ring[STAGES][NT][SC];
+  // chunks before it is used; x moves to LDS one chunk ahead of its MFMAs.
+  bf16x8_t ring[STAGES][SC];
   bf16x8_t xring[STAGES][UPT];
 #pragma unroll
   for (int st = 0; st < STAGES; ++st) {  // chunks past the end reload in-bounds data
@@ -362,133 +321,272 @@ __global__ void __launch_bounds__(256) linear_wide_kernel(LinearParams p) {
     load_x(st, xring[st]);
   }
   store_x(0, xring[0]);
-  if constexpr (PIPE) {
-    if (nchunks > 1) store_x(1, xring[1]);
-  }
   __syncthreads();
-
-  if constexpr (PIPE) {
-    // Chunk c's x sits in xs[c % 3]. Step (c, t)'s operands are read during step
-    // (c, t - 1) -- or, for t = 0, during chunk c - 1's last step, after the barrier
-    // that ended chunk c - 2 published xs[c % 3]. Chunk c stores chunk c + 2's x into
-    // xs[(c + 2) % 3], whose last reads (chunk c - 1's) all completed before the
-    // barrier that ended chunk c - 1 (the barrier waits for this wave's LDS reads).
-    auto read_b = [&](int c, int t, bf16x8_t (&b)[MT]) {
-      const bool valid = c * SC + t < total;
+  // The K range is a compile-time constant so the chunk loop unrolls completely: the
+  // compiler's wait-count pass then sees every load of the register rings in order and
+  // waits exactly for the chunk it is about to use.
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) b[mt] = valid ? xs[c % 3][mt][t][xrd[t]] : bf16x8_t{};
-    };
-    bf16x8_t b[MT];
-    read_b(0, 0, b);
+  for (int c = 0; c < nchunks; ++c) {
+    const int cur = c & 1, st = c % STAGES;
 #pragma unroll
-    for (int c0 = 0; c0 < nchunks; c0 += STAGES) {
+    for (int t = 0; t < SC; ++t) {
+      const bool valid = c * SC + t < KSTEPS;
+      const bf16x8_t a = valid ? ring[st][t] : bf16x8_t{};
 #pragma unroll
-      for (int st = 0; st < STAGES; ++st) {
-        const int c = c0 + st;
-        if (c < nchunks) {
-#pragma unroll
-          for (int t = 0; t < SC; ++t) {
-            const bool valid = c * SC + t < total;
-            const bool next = t + 1 < SC || c + 1 < nchunks;
-            bf16x8_t bn[MT];
-            if (t + 1 < SC) read_b(c, t + 1, bn);
-            else if (c + 1 < nchunks) read_b(c + 1, 0, bn);
-            // Keeps the reads above this step's MFMAs: left to itself the scheduler
-            // sinks each read below the last MFMA that uses the register it refills.
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-              const bf16x8_t a = valid ? ring[st][nt][t] : bf16x8_t{};
-#pragma unroll
-              for (int mt = 0; mt < MT; ++mt)
-                acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[mt], acc[nt][mt], 0, 0, 0);
-            }
-            if (next) {
-#pragma unroll
-              for (int mt = 0; mt < MT; ++mt) b[mt] = bn[mt];
-            }
-          }
-          if (c + STAGES < nchunks) load_w(c + STAGES, ring[st]);
-          if (c + 2 < nchunks) store_x((c + 2) % 3, xring[(st + 2) % STAGES]);
-          if (c + STAGES < nchunks) load_x(c + STAGES, xring[st]);
-          lds_barrier();
-        }
+      for (int mt = 0; mt < MT; ++mt) {
+        const bf16x8_t b = valid ? xs[cur][mt][t][xrd[t]] : bf16x8_t{};
+        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[mt], 0, 0, 0);
       }
     }
-  } else {
+    if (c + STAGES < nchunks) load_w(c + STAGES, ring[st]);
+    if (c + 1 < nchunks) store_x(cur ^ 1, xring[(st + 1) % STAGES]);
+    if (c + STAGES < nchunks) load_x(c + STAGES, xring[st]);
+    lds_barrier();
+  }
+
+  if (NTAIL && n0 + 16 * wave >= p.N) return;  // wave-uniform: a tile past N
 #pragma unroll
-    for (int c0 = 0; c0 < nchunks; c0 += STAGES) {
+  for (int mt = 0; mt < MT; ++mt) {
+    const int m = m0 + 16 * mt + (lane & 15);
+    if (m >= p.M) continue;
+    *reinterpret_cast<f32x4_t*>(p.parts + ((int64_t)ks * p.M + m) * p.N + n0 + 16 * wave + 4 * (lane >> 4)) = acc[mt];
+  }
+}
+
+template <int MT, int KSTEPS, int KSPLIT, bool NTAIL = false>
+int launch_linear_parts(LinearParams prm, hipStream_t stream) {
+  if ((NTAIL ? prm.N % 16 : prm.N % 64) || prm.K != 32 * KSTEPS * KSPLIT) return CDB_ERR_SHAPE;
+  const int n_tiles = NTAIL ? (prm.N / 16 + 3) / 4 : prm.N / 64;  // as the kernel counts
+  const int m_tiles = (prm.M + 16 * MT - 1) / (16 * MT);
+  hipLaunchKernelGGL((linear_parts_kernel<MT, KSTEPS, KSPLIT, NTAIL>),
+                     dim3((n_tiles * KSPLIT + 7) / 8 * 8 * m_tiles), dim3(256), 0, stream, prm);
+  return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
+}
+
+// ---------------------------------------------------------------------------
+// Streaming form, for every batch the row kernel above does not take. A
+// workgroup owns 16*MT rows x `consumers` * NTW column tiles (gated: gate/up
+// tile pairs) over its whole K range, and its waves have two jobs:
+//   * one producer wave moves x: chunks of SC contraction steps go straight to
+//     a ring of S LDS stages (global_load_lds, eight lanes per 128-byte row
+//     segment), S - 2 chunks ahead;
+//   * each consumer wave streams the weight tiles of its own columns from HBM
+//     into a ring of RW steps of registers and multiplies them with the staged
+//     x, every output adding its K steps in order in one accumulator (so a
+//     row's result does not depend on the tile choice or on its batch).
+// One barrier per chunk publishes a stage. What bounds the kernel is the weight
+// stream, and with it the bytes a CU pulls through its vector memory path, x
+// and weights together (about 55 B/clk for 128-byte segments; 15 B/clk for the
+// 16-row x 64-byte MFMA operand pattern, which is why x goes through LDS). Loads
+// return in order per wave: a wave that loads both kinds waits for its oldest
+// weight block, an HBM round trip, whenever it needs its newest x, so the
+// weight stream never runs ahead of x by more than x's own prefetch. With x in a
+// wave of its own the two run at their own depths. Against the form before it
+// (x loaded and stored to LDS by the waves that multiply; cold weights, us):
+//   2048 -> 6144, 200 rows            15.2 -> 12.9    100 rows  11.1 -> 10.5
+//   2048 -> 2 x 5632 gated, 200 rows  24.0 -> 19.3    100 rows  17.2 -> 14.9
+//   5632 -> 2048, 4 K ranges, 200     13.5 -> 12.0    100 rows  10.5 ->  9.1
+//   5280 -> 2 x 17920 gated, 100      118  -> 70 (5.4 TB/s of weights)
+//   5280 -> 15840, 100 rows           51   -> 40
+//   17920 -> 5280, 4 K ranges, 100    78   -> 42      256 rows   138 -> 60
+// ---------------------------------------------------------------------------
+constexpr int kStreamSteps = 4;        // SC: contraction steps per x chunk (256 bytes of a row)
+constexpr int kStreamRing = 8;         // RW: weight steps in flight per consumer wave
+constexpr int kStreamMaxConsumers = 6;
+// S: x stages in LDS. A stage is MT * SC KiB; eight row tiles fit three (and keep the
+// producer's loads in flight under the 63 a wave can count).
+template <int MT> constexpr int kStreamStages = MT < 8 ? 4 : 3;
+
+CDB_DEVICE uint32_t lds_address(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+// 16 bytes per lane from `src` to LDS at lds_base + 16 * lane (lds_base uniform over the wave).
+CDB_DEVICE void block_load_lds(const void* src, uint32_t lds_base) {
+  __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)(uintptr_t)lds_base, 16, 0, 0);
+}
+template <int N> CDB_DEVICE void wait_loads() { __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+CDB_DEVICE void meet() { __asm__ volatile("s_barrier" ::: "memory"); }
+
+// `splits` > 1 (PARTS): the workgroup covers one of `splits` equal K ranges and stores
+// fp32 partial sums to p.parts[range], for a consumer that adds them in range order and
+// rounds once (the residual RMSNorm). p.steps_per_wave holds the steps of one range.
+template <int MT, int NTW, bool GATED, bool PARTS>
+__global__ void __launch_bounds__(64 * (kStreamMaxConsumers + 1)) linear_stream_kernel(LinearParams p) {
+  constexpr int NT = GATED ? 2 * NTW : NTW;
+  constexpr int SC = kStreamSteps, RW = kStreamRing, S = kStreamStages<MT>;
+  constexpr int kUnits = 4 * SC;              // 16-byte units of one row in a chunk
+  constexpr int kRowsPerLoad = kWave / kUnits;
+  constexpr int kLoads = 16 * MT / kRowsPerLoad;  // producer loads per chunk
+  constexpr int kStage = MT * SC * 1024;
+  constexpr int kAhead = S - 2;
+  static_assert(kAhead * kLoads <= 63, "the producer's wait counts its loads in flight");
+  static_assert(RW % SC == 0 && RW % 2 == 0, "a ring turn is whole chunks, and keeps the operand buffers' parity");
+  __shared__ __attribute__((aligned(1024))) unsigned char xs[S * kStage];
+
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int consumers = blockDim.x / kWave - 1;
+  const int tiles = p.N / 16;
+  const int steps = p.steps_per_wave;
+  const int tile_steps = p.K / 32;
+
+  // Workgroups that share weights -- the row ranges of one (column range, K range) -- sit on one XCD.
+  const int col_ranges = (tiles + consumers * NTW - 1) / (consumers * NTW);
+  const int row_ranges = (p.M + 16 * MT - 1) / (16 * MT);
+  const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+  const int pair = (q / row_ranges) * 8 + xcd;
+  const int range = pair / col_ranges;
+  if (range * steps >= tile_steps) return;  // padding workgroup of the XCD-major order: exits before any barrier
+  const int m0 = (q % row_ranges) * 16 * MT;
+  const int k0 = range * steps;
+  const int chunks = (steps + SC - 1) / SC;
+
+  if (wave == consumers) {
+    // Producer. Load i covers kRowsPerLoad rows; a lane fetches the unit that belongs at its
+    // LDS slot: unit u of row r sits at slot u ^ (r % 8) within its 128-byte half, so the
+    // operand reads below (one unit of 16 rows) fall in distinct banks.
+    const char* src[kLoads];
+    int koff[kLoads];
 #pragma unroll
-      for (int st = 0; st < STAGES; ++st) {
-        const int c = c0 + st;
-        if (c < nchunks) {
-          const int cur = c & 1;
-          const bool more = c + 1 < nchunks;
+    for (int i = 0; i < kLoads; ++i) {
+      const int row = i * kRowsPerLoad + lane / kUnits, slot = lane % kUnits;
+      src[i] = reinterpret_cast<const char*>(p.x + (int64_t)min(m0 + row, p.M - 1) * p.ldx + (int64_t)k0 * 32);
+      koff[i] = ((slot & ~7) | ((slot ^ row) & 7)) * 16;
+    }
+    const uint32_t base = lds_address(xs);
+    auto issue = [&](int c) {  // units past the range's end fetch its last unit (in bounds, never read)
+      const uint32_t stage = base + (c % S) * kStage;
 #pragma unroll
-          for (int t = 0; t < SC; ++t) {
-            const bool valid = c * SC + t < total;
-            bf16x8_t b[MT];
+      for (int i = 0; i < kLoads; ++i)
+        block_load_lds(src[i] + min(c * (SC * 64) + koff[i], steps * 64 - 16), stage + i * 1024);
+    };
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) b[mt] = valid ? xs[cur][mt][t][xrd[t]] : bf16x8_t{};
+    for (int c = 0; c < kAhead; ++c)
+      if (c < chunks) issue(c);
+    // Barrier c publishes chunk c. Chunk c + kAhead goes to the stage of chunk c - 2, whose
+    // reads every consumer finished before it met barrier c - 1.
+    for (int c = 0; c < chunks; ++c) {
+      if (c + kAhead < chunks) {
+        issue(c + kAhead);
+        wait_loads<kAhead * kLoads>();
+      } else if (kAhead > 1 && c + 1 < chunks) {
+        wait_loads<kLoads>();
+      } else {
+        wait_loads<0>();
+      }
+      meet();
+    }
+    return;
+  }
+
+  const int t0 = (pair % col_ranges) * consumers * NTW + wave * NTW;
+  const char* wbase[NT];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-              const bf16x8_t a = valid ? ring[st][nt][t] : bf16x8_t{};
+  for (int j = 0; j < NTW; ++j) {
+    const int t = min(t0 + j, tiles - 1);  // past the last tile: loads it again, stores nothing
+    wbase[j] = reinterpret_cast<const char*>(p.w + ((int64_t)t * tile_steps + k0) * 512);
+    if constexpr (GATED)
+      wbase[NTW + j] = reinterpret_cast<const char*>(p.w + ((int64_t)(tiles + t) * tile_steps + k0) * 512);
+  }
+  auto load_weights = [&](int s, bf16x8_t (&w)[NT]) {
 #pragma unroll
-              for (int mt = 0; mt < MT; ++mt)
-                acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[mt], acc[nt][mt], 0, 0, 0);
-            }
-          }
-          if (c + STAGES < nchunks) load_w(c + STAGES, ring[st]);
-          if (more) store_x(cur ^ 1, xring[(st + 1) % STAGES]);
-          if (c + STAGES < nchunks) load_x(c + STAGES, xring[st]);
+    for (int nt = 0; nt < NT; ++nt)
+      w[nt] = load_w(reinterpret_cast<const bf16_t*>(wbase[nt] + (int64_t)s * 1024 + (uint32_t)(16 * lane)));
+  };
+  bf16x8_t ring[RW][NT];
+#pragma unroll
+  for (int s = 0; s < RW; ++s) load_weights(min(s, steps - 1), ring[s]);
+  f32x4_t acc[NT][MT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // This lane's operand: row lane % 16 of each row tile, k group lane / 16 of each step.
+  const int r15 = lane & 15, g = lane >> 4;
+  const bf16x8_t* const units = reinterpret_cast<const bf16x8_t*>(xs);
+  auto read_x = [&](int stage, int t, bf16x8_t (&b)[MT]) {
+    const int u = 4 * t + g;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      b[mt] = units[stage * (kStage / 16) + (16 * mt + r15) * kUnits + ((u & ~7) | ((u ^ r15) & 7))];
+  };
+  auto multiply = [&](const bf16x8_t (&w)[NT], const bf16x8_t (&b)[MT]) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[nt], b[mt], acc[nt][mt], 0, 0, 0);
+  };
+
+  // Each step's x is read while the step before it is multiplied; a chunk's last step meets
+  // the barrier that publishes the next chunk, with this wave's reads of its own stage done.
+  bf16x8_t b[2][MT];
+  meet();
+  read_x(0, 0, b[0]);
+  int stage = 0, s0 = 0;
+  // One turn of the weight ring; the blocks it loads belong to the next turn. kWhole: all of
+  // them exist, and the turn is one straight line (a branch around a load makes the compiler's
+  // later waits assume the shorter path, so only the last whole turn has them).
+  auto turn = [&](auto whole) {
+    constexpr bool kWhole = decltype(whole)::value;
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      if ((i + 1) % SC != 0) {
+        read_x(stage, (i + 1) % SC, b[(i + 1) & 1]);
+      } else {
+        stage = stage + 1 == S ? 0 : stage + 1;
+        if (kWhole || s0 + i + 1 < steps) lds_barrier();
+        read_x(stage, 0, b[(i + 1) & 1]);  // after the last step: any stage, never used
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(ring[i], b[i & 1]);
+      if (kWhole || s0 + RW + i < steps) load_weights(s0 + RW + i, ring[i]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    s0 += RW;
+  };
+  while (s0 + 2 * RW <= steps) turn(std::true_type{});
+  if (s0 + RW <= steps) turn(std::false_type{});
+#pragma unroll
+  for (int i = 0; i < RW - 1; ++i) {  // the last, partial turn
+    if (s0 + i < steps) {
+      if (s0 + i + 1 < steps) {
+        if ((i + 1) % SC == 0) {
+          stage = stage + 1 == S ? 0 : stage + 1;
           lds_barrier();
         }
+        read_x(stage, (i + 1) % SC, b[(i + 1) & 1]);
       }
+      multiply(ring[i], b[i & 1]);
     }
   }
 
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    const int m = m0 + 16 * mt + (lane & 15);
+    const int m = m0 + 16 * mt + r15;
     if (m >= p.M) continue;
-    if constexpr (KSPLIT > 1) {
-#pragma unroll
-      for (int j = 0; j < NTW; ++j) {
-        if (NTAIL && n0 + 16 * (wave * NTW + j) >= p.N) continue;  // wave-uniform: a tile past N
-        float* dst = p.parts + ((int64_t)ks * p.M + m) * p.N + n0 + 16 * (wave * NTW + j) + 4 * (lane >> 4);
-        *reinterpret_cast<f32x4_t*>(dst) = acc[j][mt];
-      }
-      continue;
-    }
 #pragma unroll
     for (int j = 0; j < NTW; ++j) {
-      if (NTAIL && n0 + 16 * (wave * NTW + j) >= p.N) continue;  // wave-uniform: a tile past N
-      Vec<bf16_t, 4> o;
+      if (t0 + j >= tiles) continue;  // wave-uniform: a tile past N
+      const int n = 16 * (t0 + j) + 4 * g;
+      if constexpr (PARTS) {
+        *reinterpret_cast<f32x4_t*>(p.parts + ((int64_t)range * p.M + m) * p.N + n) = acc[j][mt];
+      } else {
+        Vec<bf16_t, 4> o;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if constexpr (GATED) {
-          const float gate = round_bf16(acc[j][mt][i]);
-          const float act = silu_bf16(gate);
-          o.set(i, act * round_bf16(acc[NTW + j][mt][i]));
-        } else {
-          o.set(i, acc[j][mt][i]);
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (GATED) {
+            const float act = silu_bf16(round_bf16(acc[j][mt][i]));
+            o.set(i, act * round_bf16(acc[NTW + j][mt][i]));
+          } else {
+            o.set(i, acc[j][mt][i]);
+          }
         }
+        o.store(p.y + (int64_t)m * p.ldy + n);
       }
-      o.store(p.y + (int64_t)m * p.ldy + n0 + 16 * (wave * NTW + j) + 4 * (lane >> 4));
     }
   }
-}
-
-template <int MT, int NTW, int SC, int STAGES, bool GATED, int KSTEPS, int KSPLIT = 1, bool NTAIL = false,
-          bool PIPE = false>
-int launch_linear_wide(LinearParams prm, hipStream_t stream) {
-  if ((NTAIL ? prm.N % 16 : prm.N % (64 * NTW)) || prm.K != 32 * KSTEPS * KSPLIT) return CDB_ERR_SHAPE;
-  const int n_tiles = NTAIL ? (prm.N / 16 + 4 * NTW - 1) / (4 * NTW) : prm.N / (64 * NTW);  // as the kernel counts
-  const int m_tiles = (prm.M + 16 * MT - 1) / (16 * MT);
-  const int pairs = n_tiles * KSPLIT;
-  hipLaunchKernelGGL((linear_wide_kernel<MT, NTW, SC, STAGES, GATED, KSTEPS, KSPLIT, NTAIL, PIPE>),
-                     dim3((pairs + 7) / 8 * 8 * m_tiles), dim3(256), 0, stream, prm);
-  return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
 }
 
 // W [rows, K] (row stride ldw) -> packed MFMA operand order; one thread per 16 bytes.
@@ -591,8 +689,8 @@ __global__ void __launch_bounds__(kArgmaxMergeThreads) linear_argmax_merge_kerne
 // Launch shape of one instantiation: threads per workgroup are capped so the
 // accumulators and a batch of loads fit without spilling, and the LDS partial
 // tiles (SLOTS x NT x MT x 1 KiB) stay within 64 KiB.
-template <int MT, int NB, int S, bool GATED> struct LinearShape {
-  static constexpr int kNT = GATED ? 2 * NB : NB;
+template <int MT, int NB, int S> struct LinearShape {
+  static constexpr int kNT = NB;
   static constexpr int kRegs = 4 * (kNT * S + MT * S + kNT * MT);
   static constexpr int kThreads = kRegs <= 96 ? 1024 : 512;
   static constexpr int kSlots = 64 / (kNT * MT) < 8 ? 64 / (kNT * MT) : 8;
@@ -607,14 +705,14 @@ inline int linear_steps_per_wave(int32_t in_features, int batch, int max_waves) 
   return (per_wave + batch - 1) / batch * batch;
 }
 
-template <int MT, int NB, int S, bool GATED, bool ARGMAX = false>
+template <int MT, int NB, int S, bool ARGMAX = false>
 int launch_linear(LinearParams prm, hipStream_t stream, int max_waves = kLinearMaxWaves) {
-  using Shape = LinearShape<MT, NB, S, GATED>;
+  using Shape = LinearShape<MT, NB, S>;
   if (prm.N % (16 * NB)) return CDB_ERR_SHAPE;
   const int waves_cap = max_waves < Shape::kMaxWaves ? max_waves : Shape::kMaxWaves;
   prm.steps_per_wave = linear_steps_per_wave(prm.K, S, waves_cap);
   const int nwaves = (prm.K / 32 + prm.steps_per_wave - 1) / prm.steps_per_wave;
-  hipLaunchKernelGGL((linear_kernel<MT, NB, S, Shape::kSlots, GATED, Shape::kThreads, ARGMAX>),
+  hipLaunchKernelGGL((linear_kernel<MT, NB, S, Shape::kSlots, Shape::kThreads, ARGMAX>),
                      dim3(prm.N / (16 * NB)), dim3(nwaves * kWave), 0, stream, prm);
   return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
 }
@@ -625,53 +723,95 @@ using namespace cdb;
 
 namespace {
 
-// Tile choice, from a sweep over (NB, S, waves) at the Ouro-1.4B and Huginn-0125
-// projection shapes with cold weights: two column tiles per workgroup once N is
-// wide enough to keep more than 128 workgroups; otherwise one, so N = 2048
-// still spreads over 128 CUs. Batches of 4 steps (2 at four row tiles, for
-// registers); 8 waves per workgroup for one row tile, 4 above.
+// The row kernel's tile choice, from a sweep over (NB, S, waves) at the Ouro-1.4B
+// and Huginn-0125 projection shapes with cold weights: two column tiles per
+// workgroup once N is wide enough to keep more than 128 workgroups; otherwise
+// one, so N = 2048 still spreads over 128 CUs. Batches of 4 steps (2 at four row
+// tiles, for registers); 8 waves per workgroup for one row tile, 4 above.
 template <int MT, int S>
-int dispatch_rows(const LinearParams& prm, bool gated, int max_waves, hipStream_t stream) {
-  const bool wide = prm.N >= 4096 && prm.N % 32 == 0;
-  if (wide) {
-    return gated ? launch_linear<MT, 2, S, true>(prm, stream, max_waves)
-                 : launch_linear<MT, 2, S, false>(prm, stream, max_waves);
-  }
-  return gated ? launch_linear<MT, 1, S, true>(prm, stream, max_waves)
-               : launch_linear<MT, 1, S, false>(prm, stream, max_waves);
+int dispatch_rows(const LinearParams& prm, int max_waves, hipStream_t stream) {
+  return prm.N >= 4096 && prm.N % 32 == 0 ? launch_linear<MT, 2, S>(prm, stream, max_waves)
+                                          : launch_linear<MT, 1, S>(prm, stream, max_waves);
 }
 
-// Wide-tile path: batches of 33 to 256 rows over 2048-wide inputs with outputs
-// of 4096+ columns (the Ouro-1.4B QKV and gate/up projections). Tiles from a
-// sweep over (row tiles, column tiles, chunk, stages, pipelined x reads) with
-// cold weights; the pipelined form wins only where a wave has 16 or more MFMAs
-// per step to hide its reads behind (the gated projection above 64 rows).
+enum class StreamMode { kPlain, kGated, kParts };
+
+struct StreamTile {
+  int mt, ntw, consumers;  // row tiles, column tiles per consumer wave, consumer waves
+};
+
+template <int MT, int NTW, bool GATED, bool PARTS>
+int launch_stream(LinearParams prm, const StreamTile& t, int splits, hipStream_t stream) {
+  prm.steps_per_wave = prm.K / 32 / splits;
+  const int cols = t.consumers * NTW;
+  const int64_t pairs = (int64_t)((prm.N / 16 + cols - 1) / cols) * splits;
+  const int64_t row_ranges = (prm.M + 16 * MT - 1) / (16 * MT);
+  hipLaunchKernelGGL((linear_stream_kernel<MT, NTW, GATED, PARTS>), dim3((unsigned)((pairs + 7) / 8 * 8 * row_ranges)),
+                     dim3((t.consumers + 1) * kWave), 0, stream, prm);
+  return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
+}
+
+template <int MT>
+int launch_stream_rows(const LinearParams& prm, const StreamTile& t, StreamMode mode, int splits, hipStream_t stream) {
+  if (mode == StreamMode::kGated) return launch_stream<MT, 1, true, false>(prm, t, splits, stream);
+  if (mode == StreamMode::kPlain)
+    return t.ntw == 2 ? launch_stream<MT, 2, false, false>(prm, t, splits, stream)
+                      : launch_stream<MT, 1, false, false>(prm, t, splits, stream);
+  return t.ntw == 2 ? launch_stream<MT, 2, false, true>(prm, t, splits, stream)
+                    : launch_stream<MT, 1, false, true>(prm, t, splits, stream);
+}
+
+// The tile that makes the busiest CU pull the fewest bytes: workgroups are dealt evenly over
+// 256 CUs, so a CU runs ceil(workgroups / 256) of them, and each pulls its rows of x and its
+// columns of W once per contraction step. Against a sweep of every tile over the Ouro-1.4B and
+// Huginn-0125 shapes from 1 to 256 rows the choice is within 4% of the best one (200 rows,
+// 2048 -> 2 x 5632 gated: chosen 112 rows x 3 tile pairs, 236 workgroups, 18.3 us; 112 x 4,
+// 176 workgroups, 19.7; 64 x 3, 472 workgroups, 24).
+StreamTile choose_stream_tile(const LinearParams& prm, StreamMode mode, int splits) {
+  const int row_tiles = (prm.M + 15) / 16, col_tiles = prm.N / 16;
+  StreamTile best{1, 1, 1};
+  int64_t best_cost = INT64_MAX;
+  for (int mt = 1; mt <= 8 && mt <= row_tiles; ++mt) {
+    for (int ntw = 1; ntw <= (mode == StreamMode::kGated ? 1 : 2); ++ntw) {
+      for (int c = 2; c <= kStreamMaxConsumers; ++c) {
+        const int cols = c * ntw;
+        if (ntw == 2 && cols <= kStreamMaxConsumers) continue;  // one tile per wave covers it
+        const int64_t groups = (int64_t)((col_tiles + cols - 1) / cols) * splits * ((row_tiles + mt - 1) / mt);
+        const int64_t cost = (groups + 255) / 256 * (mt + cols * (mode == StreamMode::kGated ? 2 : 1));
+        if (cost <= best_cost) {  // a tie goes to the taller tile: fewer row ranges re-read W from L2
+          best_cost = cost;
+          best = StreamTile{mt, ntw, c};
+        }
+      }
+    }
+  }
+  return best;
+}
+
+int dispatch_stream(const LinearParams& prm, StreamMode mode, int splits, hipStream_t stream) {
+  const StreamTile t = choose_stream_tile(prm, mode, splits);
+  switch (t.mt) {
+    case 1: return launch_stream_rows<1>(prm, t, mode, splits, stream);
+    case 2: return launch_stream_rows<2>(prm, t, mode, splits, stream);
+    case 3: return launch_stream_rows<3>(prm, t, mode, splits, stream);
+    case 4: return launch_stream_rows<4>(prm, t, mode, splits, stream);
+    case 5: return launch_stream_rows<5>(prm, t, mode, splits, stream);
+    case 6: return launch_stream_rows<6>(prm, t, mode, splits, stream);
+    case 7: return launch_stream_rows<7>(prm, t, mode, splits, stream);
+    default: return launch_stream_rows<8>(prm, t, mode, splits, stream);
+  }
+}
+
+// Shapes cdb_linear takes above 64 rows: 2048-wide inputs with outputs of 4096+ columns
+// (the Ouro-1.4B QKV and gate/up projections) up to 256 rows, 5280-wide ones (Huginn) up to 128.
 bool wide_path(const LinearParams& prm) {
-  // 5280-wide inputs (the Huginn QKV and gate/up projections) between 65 and 128 rows.
   if (prm.K == 5280) return prm.M > 64 && prm.M <= 128 && prm.N >= 4096 && prm.N % 16 == 0;
   return prm.M > 32 && prm.M <= kLinearWideMaxRows && prm.K == 2048 && prm.N >= 4096 && prm.N % 128 == 0;
 }
 
-int dispatch_wide(const LinearParams& prm, bool gated, hipStream_t stream) {
-  if (prm.K == 5280) {  // 128-row tiles, from a cold-weight sweep at 64-128 rows
-    return gated ? launch_linear_wide<8, 1, 2, 4, true, 165, 1, true>(prm, stream)
-                 : launch_linear_wide<8, 1, 2, 4, false, 165, 1, true>(prm, stream);
-  }
-  if (prm.M <= 64) {
-    return gated ? launch_linear_wide<2, 1, 4, 4, true, 64>(prm, stream)
-                 : launch_linear_wide<2, 1, 4, 4, false, 64>(prm, stream);
-  }
-  if (prm.M <= 128) {
-    return gated ? launch_linear_wide<4, 1, 2, 4, true, 64, 1, false, true>(prm, stream)
-                 : launch_linear_wide<4, 1, 2, 4, false, 64>(prm, stream);
-  }
-  return gated ? launch_linear_wide<8, 1, 2, 4, true, 64, 1, false, true>(prm, stream)
-               : launch_linear_wide<4, 2, 2, 4, false, 64>(prm, stream);
-}
-
-// Split-K form: 2048- and 5632-wide inputs into outputs of a multiple of 64
+// Split-K projections: 2048- and 5632-wide inputs into outputs of a multiple of 64
 // columns (the Ouro O and down projections), fp32 partials per K range. Split
-// counts and tiles from a sweep with cold weights, timed together with the
+// counts from a sweep with cold weights, timed together with the
 // residual RMSNorm that adds the partials: four ranges up to 64 rows; above,
 // two for the 2048-wide input (whose partials would cost more than the
 // parallelism buys) up to 128 rows, four for the 5632-wide one up to 256. The
@@ -693,36 +833,35 @@ int parts_splits(int64_t rows, int32_t out_features, int32_t in_features) {
   return 0;
 }
 
-int dispatch_parts(const LinearParams& prm, hipStream_t stream) {
-  if (prm.K == 2048) {
-    if (prm.M <= 32) return launch_linear_wide<1, 1, 4, 4, false, 16, 4>(prm, stream);
-    if (prm.M <= 64) return launch_linear_wide<2, 1, 4, 4, false, 16, 4>(prm, stream);
-    return launch_linear_wide<2, 1, 4, 4, false, 32, 2>(prm, stream);
-  }
-  if (prm.K == 5632) {
-    if (prm.M <= 16) return launch_linear_wide<1, 1, 4, 4, false, 22, 8>(prm, stream);
-    if (prm.M <= 32) return launch_linear_wide<1, 1, 4, 4, false, 44, 4>(prm, stream);
-    if (prm.M <= 64) return launch_linear_wide<2, 1, 4, 4, false, 44, 4>(prm, stream);
-    if (prm.M <= 128) return launch_linear_wide<4, 1, 2, 4, false, 44, 4>(prm, stream);
-    return launch_linear_wide<8, 1, 2, 4, false, 44, 4, false, true>(prm, stream);  // two row ranges, pipelined
-  }
-  if (prm.K == 5280) {
-    if (prm.M <= 16) return launch_linear_wide<1, 1, 4, 4, false, 55, 3, true>(prm, stream);
-    return launch_linear_wide<4, 1, 2, 4, false, 55, 3, true>(prm, stream);
-  }
-  if (prm.K == 17920) {
-    if (prm.M <= 16) return launch_linear_wide<1, 1, 4, 4, false, 70, 8, true>(prm, stream);
-    if (prm.M <= 64) return launch_linear_wide<4, 1, 2, 4, false, 70, 8, true>(prm, stream);
-    return launch_linear_wide<4, 1, 2, 4, false, 140, 4, true>(prm, stream);
-  }
-  return CDB_ERR_SHAPE;
+// The few-row form where it measured faster (figures at its kernel); from the next width up the
+// streaming form is: 2048 -> 2048 at 90 rows 5.8 -> 5.5 us, 5632 -> 2048 at 90 / 200 rows
+// 9.1 -> 8.9 / 13.5 -> 12.0, 5280 -> 5280 at 100 rows 23.1 -> 17.1, 17920 -> 5280 at
+// 32 / 100 rows 38.6 -> 34.1 / 78 -> 42.
+int dispatch_parts(const LinearParams& prm, int splits, hipStream_t stream) {
+  if (prm.K == 2048 && prm.M <= 32) return launch_linear_parts<1, 16, 4>(prm, stream);
+  if (prm.K == 2048 && prm.M <= 64) return launch_linear_parts<2, 16, 4>(prm, stream);
+  if (prm.K == 5632 && prm.M <= 16) return launch_linear_parts<1, 22, 8>(prm, stream);
+  if (prm.K == 5632 && prm.M <= 32) return launch_linear_parts<1, 44, 4>(prm, stream);
+  if (prm.K == 5632 && prm.M <= 64) return launch_linear_parts<2, 44, 4>(prm, stream);
+  if (prm.K == 5280 && prm.M <= 16) return launch_linear_parts<1, 55, 3, true>(prm, stream);
+  if (prm.K == 17920 && prm.M <= 16) return launch_linear_parts<1, 70, 8, true>(prm, stream);
+  return dispatch_stream(prm, StreamMode::kParts, splits, stream);
+}
+
+// The row kernel's share of up to 32 rows: plain projections of fewer than 8192 columns up to
+// 16 rows (2048 -> 6144 at 1 / 13 rows 6.4 / 7.1 us against 7.9 / 8.0 streamed, 10560 -> 5280 at
+// 16 rows 26 against 31; from 5280 -> 15840 on the streaming form wins, 29.1 against 31.8 at 16
+// rows), and the LM heads, whose logits then equal those of the argmax form bit for bit.
+// Gated projections stream at every batch: 2048 -> 2 x 5632 at 16 rows 11.4 -> 10.0 us,
+// 5280 -> 2 x 17920 72 -> 61 us.
+bool use_row_kernel(const LinearParams& prm, bool gated) {
+  return !gated && (prm.M <= 16 ? prm.N < 8192 || prm.N > 16384 : prm.M <= 32 && prm.N > 16384);
 }
 
 int dispatch_linear(const LinearParams& prm, bool gated, hipStream_t stream) {
-  if (wide_path(prm)) return dispatch_wide(prm, gated, stream);
-  if (prm.M <= 16) return dispatch_rows<1, 4>(prm, gated, 8, stream);
-  if (prm.M <= 32) return dispatch_rows<2, 4>(prm, gated, 4, stream);
-  return dispatch_rows<4, 2>(prm, gated, 4, stream);
+  if (use_row_kernel(prm, gated))
+    return prm.M <= 16 ? dispatch_rows<1, 4>(prm, 8, stream) : dispatch_rows<2, 4>(prm, 4, stream);
+  return dispatch_stream(prm, gated ? StreamMode::kGated : StreamMode::kPlain, 1, stream);
 }
 
 }  // namespace
@@ -793,7 +932,7 @@ extern "C" int cdb_linear_parts(const void* x, int64_t ldx, const void* w_packed
   prm.N = out_features;
   prm.K = in_features;
   prm.steps_per_wave = 0;
-  return dispatch_parts(prm, stream);
+  return dispatch_parts(prm, splits, stream);
 }
 
 extern "C" int64_t cdb_linear_argmax_workspace_bytes(int32_t rows, int32_t out_features) {
@@ -833,11 +972,11 @@ extern "C" int cdb_linear_argmax(const void* x, int64_t ldx, const void* w_packe
   const bool two = out_features >= 4096 && out_features % 32 == 0;
   int rc;
   if (rows <= 16)
-    rc = two ? launch_linear<1, 2, 4, false, true>(prm, stream, 8) : launch_linear<1, 1, 4, false, true>(prm, stream, 8);
+    rc = two ? launch_linear<1, 2, 4, true>(prm, stream, 8) : launch_linear<1, 1, 4, true>(prm, stream, 8);
   else if (rows <= 32)
-    rc = two ? launch_linear<2, 2, 4, false, true>(prm, stream, 4) : launch_linear<2, 1, 4, false, true>(prm, stream, 4);
+    rc = two ? launch_linear<2, 2, 4, true>(prm, stream, 4) : launch_linear<2, 1, 4, true>(prm, stream, 4);
   else
-    rc = two ? launch_linear<4, 2, 2, false, true>(prm, stream, 4) : launch_linear<4, 1, 2, false, true>(prm, stream, 4);
+    rc = two ? launch_linear<4, 2, 2, true>(prm, stream, 4) : launch_linear<4, 1, 2, true>(prm, stream, 4);
   if (rc != CDB_OK) return rc;
   ArgmaxEmbed emb{static_cast<const bf16_t*>(embed), static_cast<bf16_t*>(bank), bank_slots, out_features,
                   bank_rows, width};

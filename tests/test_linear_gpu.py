@@ -253,6 +253,52 @@ def test_wide_tile_forms_give_a_row_the_same_bits_in_any_batch() -> None:
     assert ((gated[256].float() - ref).abs() <= 2 * _bf16_ulp(ref) + 1e-3).float().mean().item() >= 0.99
 
 
+@pytest.mark.parametrize("rows", [17, 33, 64])
+@pytest.mark.parametrize("k", [32, 96, 256, 288, 512, 544])
+@pytest.mark.parametrize("n", [16, 112])
+def test_streaming_form_at_ring_and_tile_edges(rows: int, k: int, n: int) -> None:
+    """K of 1, 3, 8, 9, 16 and 17 contraction steps (part of a chunk, part of a weight ring turn,
+    whole turns, one step more), 1 and 7 column tiles (a workgroup's last waves have none), rows
+    one past a tile, from a strided x and into a strided y: plain and gated."""
+
+    from continuous_depth_batching_amd import ops
+
+    x_big, w = _inputs(rows, 2 * k, 2 * n, seed=rows + 3 * k + n)
+    x, w = x_big[:, k:], w[:, :k].contiguous()
+    y_big = torch.full((rows, n + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.linear_raw(x, ops.pack_linear_weight(w[:n]), y_big[:, :n])
+    act = torch.empty((rows, n), dtype=torch.bfloat16, device="cuda")
+    ops.linear_raw(x, ops.pack_linear_weight(w), act, gated=True)
+    torch.cuda.synchronize()
+    assert (y_big[:, n:] == 7.0).all()
+    full, err = x.float() @ w.float().t(), _sum_error(x, w)
+    _check_rounded(y_big[:, :n], full[:, :n], max_mismatch=0.02, extra=err[:, :n])
+    gu = full.bfloat16().float()
+    g, u = gu[:, :n], gu[:, n:]
+    a = (g * torch.sigmoid(g)).bfloat16().float()
+    dg, du = _bf16_ulp(g) + err[:, :n], _bf16_ulp(u) + err[:, n:]
+    _check_rounded(act, a * u, max_mismatch=0.03, extra=1.1 * u.abs() * dg + (a.abs() + dg) * du)
+
+
+@pytest.mark.parametrize("rows,k,n", [(17, 5280, 5280), (81, 5280, 80), (113, 17920, 1296), (129, 5632, 2048),
+                                      (225, 17920, 112)])
+def test_streamed_partials_at_row_range_edges(rows: int, k: int, n: int) -> None:
+    """Row counts one past a row range, K ranges of 55, 140 and 44 steps, wide and narrow outputs:
+    every partial against its range's fp32 product (the bound of the test above)."""
+
+    from continuous_depth_batching_amd import ops
+
+    splits = ops.linear_parts_splits(rows, n, k)
+    x, w = _inputs(rows, k, n, seed=rows + k + n)
+    parts = torch.full((splits, rows, n), float("nan"), device="cuda")
+    ops.linear_parts_raw(x, ops.pack_linear_weight(w), parts)
+    torch.cuda.synchronize()
+    width = k // splits
+    for s in range(splits):
+        xs, ws = x[:, s * width:(s + 1) * width].float(), w[:, s * width:(s + 1) * width].float()
+        assert ((parts[s] - xs @ ws.t()).abs() <= (xs.abs() @ ws.abs().t()) * 2.0 ** -16).all()
+
+
 @pytest.mark.parametrize("rows,k,n", [(1, 2048, 2048), (16, 5632, 2048), (33, 2048, 2048), (96, 5632, 2048),
                                       (128, 2048, 2048), (256, 5632, 2048), (7, 5280, 5280), (128, 17920, 5280)])
 def test_norm_from_partials_is_the_two_step_result(rows: int, k: int, n: int) -> None:
