@@ -212,7 +212,19 @@ CDB_DEVICE void block_load_lds(const void* src, uint32_t lds_base) {
   __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)(uintptr_t)lds_base, 16, 0, 0);
 }
 
-template <int D>
+// Scalar load of a word that no kernel writes while this one runs (the address is wave-uniform).
+typedef __attribute__((address_space(4))) const int32_t const_int32;
+CDB_DEVICE int load_uniform(const int32_t* p, int i) { return ((const const_int32*)p)[i]; }
+
+// kPages16: pages of 16 tokens or more. The rows of one block load (4 or 8 consecutive
+// keys, aligned) then share a page, so its block id is wave-uniform: it is read with a
+// scalar load one block ahead, and the load's address is a scalar base plus a lane
+// offset. (Looked up per lane in an LDS copy of the table, each load stalled its wave for
+// an LDS round trip and cost some 35 vector instructions, 70 a block, as many as the
+// softmax: 24 prompts of 24-1300 tokens, 16 heads x 128, 59.5 -> 49.8 us.)
+// Smaller pages keep the per-lane lookup, and so do heads of 96, whose block loads leave a
+// quarter of their lanes out: 64 prompts of such heads took 52.5 us with it and 53.2 without.
+template <int D, bool kPages16>
 __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillParams P) {
   using L = BlockLayout<D>;
   constexpr int kStages = 3;               // key blocks resident: computing b, in flight b+1 and b+2
@@ -224,7 +236,7 @@ __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillPara
 
   // Stage s: K image at s * 2 * kBytes, V image right after it.
   __shared__ __attribute__((aligned(1024))) unsigned char ring[kStages * 2 * L::kBytes];
-  __shared__ int page_lds[kLdsPages];
+  __shared__ int page_lds[kPages16 ? 1 : kLdsPages];
 
   // One workgroup per (tile, head), heads fastest: the host lists the tiles
   // longest prefix first, so the heaviest workgroups of every head start first.
@@ -232,7 +244,7 @@ __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillPara
   const int h = blockIdx.x - tile * P.num_heads;
   if (tile >= P.num_tiles) return;
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int col = lane & 31;   // query column of S^T / O^T, or row of an A operand
   const int half = lane >> 5;  // k-slice half of the operands
@@ -282,7 +294,7 @@ __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillPara
   // The block ids' loads overlap Q's; both have landed before the first block
   // load is issued (loads and stores of different kinds need not complete in
   // order, so the block-load waits below count block loads alone).
-  fill_page_table(P, g, page_lds);
+  if constexpr (!kPages16) fill_page_table(P, g, page_lds);
   __asm__ volatile("s_waitcnt vmcnt(0)" : "+v"(q_raw[0])::"memory");
 #pragma unroll
   for (int c = 0; c < kQSteps; ++c) {
@@ -299,6 +311,22 @@ __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillPara
   const uint32_t page_base = lds_address(page_lds);
   const int bs_mask = (1 << P.block_size_log2) - 1;
   const int64_t row_elems = (int64_t)P.num_kv_heads * D;
+  // kPages16: load i's rows start at first_row(b, i); rows past key_end - 1 repeat that row,
+  // which lies in the page of the load's first row or, when that row is past it too, in its own.
+  int next_ids[L::kWaveLoads];  // block ids of the next block to issue
+  const uint32_t block_limit = (uint32_t)min(P.pool_blocks, (int64_t)0x7fffffff);
+  const uint32_t row_bytes = (uint32_t)(row_elems * (int)sizeof(bf16_t));  // a page is under 2^31 bytes
+  const uint32_t page_bytes = row_bytes << P.block_size_log2;
+  const uint32_t head_bytes = (uint32_t)(g.kvh * D) * (uint32_t)sizeof(bf16_t);
+  auto first_row = [&](int b, int i) { return min(b * kKeys + (4 * i + wave) * (64 / L::kRowChunks), g.key_end - 1); };
+  auto fetch_ids = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < L::kWaveLoads; ++i) {
+      // Used one block later, so that nothing waits for it here; a prefix longer than the
+      // table (malformed) reads its last entry: in bounds, values unspecified.
+      next_ids[i] = load_uniform(g.table, max(min(first_row(b, i) >> P.block_size_log2, P.table_width - 1), 0));
+    }
+  };
   auto issue_block = [&](int b) {
     if (b >= num_blocks) return;
     const uint32_t k_img = ring_lds + (b % kStages) * 2 * L::kBytes;
@@ -306,6 +334,25 @@ __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillPara
     // keeps them from being hoisted into registers held across the loop).
     int ln = lane;
     __asm__ volatile("" : "+v"(ln));
+    if constexpr (kPages16) {
+#pragma unroll
+      for (int i = 0; i < L::kWaveLoads; ++i) {
+        const int row = (4 * i + wave) * (64 / L::kRowChunks) + ln / L::kRowChunks;
+        const int chunk = (ln % L::kRowChunks) ^ (2 * L::sub(row));
+        // An unmapped page (a malformed table) reads block 0: in bounds, values unspecified.
+        const uint32_t blk = (uint32_t)next_ids[i] < block_limit ? (uint32_t)next_ids[i] : 0u;
+        const uint64_t base = (uint64_t)blk * page_bytes + head_bytes;
+        const uint32_t in_page = (uint32_t)(min(b * kKeys + row, g.key_end - 1) & bs_mask);
+        const uint32_t off = in_page * row_bytes + (uint32_t)chunk * 16u;
+        const uint32_t dst = k_img + (4 * i + wave) * 1024;
+        if (L::kChunks == L::kRowChunks || chunk < L::kChunks) {
+          block_load_lds(reinterpret_cast<const char*>(k_base) + base + off, dst);
+          block_load_lds(reinterpret_cast<const char*>(v_base) + base + off, dst + L::kBytes);
+        }
+      }
+      fetch_ids(b + 1);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < L::kWaveLoads; ++i) {
       const int slot_index = (4 * i + wave) * 64 + ln;
@@ -325,6 +372,7 @@ __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillPara
       }
     }
   };
+  if constexpr (kPages16) fetch_ids(block0);
 
   // Operand addresses within a stage. S^T: row `col`, logical chunk 2c + half
   // -> byte col * kRowBytes + ((c ^ sub) * 2 + half) * 16. V^T (transpose loads,
@@ -446,10 +494,22 @@ __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillPara
       o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pb[t], o[j], 0, 0, 0);
     }
   };
+  // Parts of split tiles all start together, a full GPU of equal work; the scheduler prefers a
+  // SIMD's oldest wave, so its workgroups finish one after the other and the last run alone.
+  // A part's priority falls with the blocks it has left, which keeps the workgroups of a CU
+  // abreast (4 x 128 queries after 16,000 keys: 123 -> 118 us). Whole tiles, of all lengths,
+  // are refilled from the rest of the launch and do not gain (49.7 -> 50.7 us).
+  auto set_priority = [&](int left) {
+    if (slot < 0) return;
+    if (left >= 24) __builtin_amdgcn_s_setprio(3);
+    else if (left >= 12) __builtin_amdgcn_s_setprio(2);
+    else if (left >= 4) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+  };
   constexpr int kJ0 = 1;  // V^T tiles read during the softmax; the rest after the first P V
   auto stage_lds = [&](int b) { return ring_lds + (b % kStages) * 2 * L::kBytes; };
 
-  lds_barrier();  // page_lds
+  if constexpr (!kPages16) lds_barrier();  // page_lds
   for (int i = 0; i < kStages - 1; ++i) issue_block(block0 + i);
   // The first block landed once at most the second block's loads are outstanding.
   if (num_blocks > block0 + 1) {
@@ -457,7 +517,10 @@ __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillPara
   } else {
     __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  set_priority(num_blocks - block0);
   for (int b = block0; b < num_blocks; ++b) {
+    const int left = num_blocks - b;
+    if (left == 23 || left == 11 || left == 3) set_priority(left);
     // Block b has landed once at most block b + 1's loads are outstanding.
     if (b > block0) {
       if (b + 1 < num_blocks) {
@@ -859,7 +922,16 @@ int launch(const void* kernel, int64_t groups, const PrefillParams& P, hipStream
   return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
 }
 
-template <int D> const void* bf16_kernel() { return reinterpret_cast<const void*>(&prefill_attention_bf16_kernel<D>); }
+// Pages of 16 tokens or more (and under 2 GiB, for 32-bit offsets inside one) have one block id
+// per block load; heads of 96 keep the per-lane lookup (see the kernel).
+template <int D> const void* bf16_kernel(const PrefillParams& P) {
+  if constexpr (D != 96) {
+    if (P.block_size_log2 >= 4 && P.table_width > 0 &&
+        ((int64_t)P.num_kv_heads * D * 2 << P.block_size_log2) < ((int64_t)1 << 31))
+      return reinterpret_cast<const void*>(&prefill_attention_bf16_kernel<D, true>);
+  }
+  return reinterpret_cast<const void*>(&prefill_attention_bf16_kernel<D, false>);
+}
 template <int D> const void* f32_kernel() { return reinterpret_cast<const void*>(&prefill_attention_f32_kernel<D>); }
 template <int D> const void* merge_kernel() { return reinterpret_cast<const void*>(&prefill_merge_kernel<D>); }
 
@@ -887,9 +959,9 @@ int cdb_prefill_attention(const void* q, const void* k_pool, const void* v_pool,
   if (dtype == CDB_DTYPE_BF16) {
     const int64_t groups = (int64_t)num_tiles * num_heads;
     switch (head_dim) {
-      case 64: return launch(bf16_kernel<64>(), groups, P, stream);
-      case 96: return launch(bf16_kernel<96>(), groups, P, stream);
-      case 128: return launch(bf16_kernel<128>(), groups, P, stream);
+      case 64: return launch(bf16_kernel<64>(P), groups, P, stream);
+      case 96: return launch(bf16_kernel<96>(P), groups, P, stream);
+      case 128: return launch(bf16_kernel<128>(P), groups, P, stream);
       default: return CDB_ERR_UNSUPPORTED;
     }
   }
@@ -939,13 +1011,13 @@ int cdb_prefill_attention_split(const void* q, const void* k_pool, const void* v
   int code = CDB_ERR_UNSUPPORTED;
   switch (head_dim) {
     case 64:
-      code = launch(bf16_kernel<64>(), groups, P, stream);
+      code = launch(bf16_kernel<64>(P), groups, P, stream);
       return code == CDB_OK ? launch(merge_kernel<64>(), merge_groups, P, stream) : code;
     case 96:
-      code = launch(bf16_kernel<96>(), groups, P, stream);
+      code = launch(bf16_kernel<96>(P), groups, P, stream);
       return code == CDB_OK ? launch(merge_kernel<96>(), merge_groups, P, stream) : code;
     case 128:
-      code = launch(bf16_kernel<128>(), groups, P, stream);
+      code = launch(bf16_kernel<128>(P), groups, P, stream);
       return code == CDB_OK ? launch(merge_kernel<128>(), merge_groups, P, stream) : code;
   }
   return code;

@@ -311,6 +311,54 @@ def test_exit_kv_copy_bit_exact() -> None:
     np.testing.assert_array_equal(host(pt), want)
 
 
+@pytest.mark.parametrize("head_dim", [64, 96, 128])
+@pytest.mark.parametrize("split", [False, True])
+def test_prefill_attention_does_not_depend_on_the_page_size(head_dim: int, split: bool) -> None:
+    """The same keys and values paged by 4 tokens (block ids looked up per lane) and by 16, 32 and
+    128 (one block id per block load): the outputs agree bit for bit, for whole tiles and for
+    tiles split over workgroups, at lengths around a key block, a tile and a page."""
+
+    from continuous_depth_batching_amd import ops
+
+    rng = np.random.default_rng(head_dim)
+    heads, kv_heads, lens = 4, 2, np.array([1, 31, 33, 129, 200], np.int64)
+    pasts = np.array([0, 33, 5, 96, 700], np.int64)
+    totals = pasts + lens
+    q = dev(rng.standard_normal((int(lens.sum()), heads, head_dim)).astype(np.float32), torch.bfloat16)
+    kv = [dev(rng.standard_normal((2, int(n), kv_heads, head_dim)).astype(np.float32), torch.bfloat16) for n in totals]
+    i32 = lambda a: dev(np.ascontiguousarray(a, dtype=np.int32))
+    cu, past, trow = i32(np.concatenate([[0], np.cumsum(lens)])), i32(pasts), i32(np.arange(lens.size))
+    tile_seq, tile_q0 = (i32(t) for t in ops.prefill_tiles(lens, pasts))
+    work = ops.prefill_split_work(lens, pasts, num_heads=heads, max_blocks=8)
+    partials = torch.empty(ops.prefill_partial_bytes(work.num_slots, heads, head_dim) // 4, device="cuda")
+    got = {}
+    for bs in (4, 16, 32, 128):
+        pages = (totals + bs - 1) // bs
+        perm = rng.permutation(int(pages.sum())).astype(np.int32)
+        table = np.full((lens.size, int(pages.max())), -1, np.int32)
+        pool = torch.full((1, 2, int(pages.sum()) * bs, kv_heads, head_dim), float("nan"), dtype=torch.bfloat16,
+                          device="cuda")
+        at = 0
+        for s, n in enumerate(pages):
+            table[s, :n] = perm[at:at + n]
+            at += int(n)
+            t = np.arange(int(totals[s]))
+            pool[0][:, torch.from_numpy(table[s, t // bs].astype(np.int64) * bs + t % bs).cuda()] = kv[s]
+        out = torch.full_like(q, 7.0)
+        view = ops.KVPoolView(pool, bs)
+        if split:
+            ops.prefill_attention_split_raw(q, view, 0, i32(table), trow, cu, past, i32(work.items), i32(work.merges),
+                                            work.num_slots, partials, out, head_dim ** -0.5)
+        else:
+            ops.prefill_attention_raw(q, view, 0, i32(table), trow, cu, past, tile_seq, tile_q0, out,
+                                      head_dim ** -0.5)
+        got[bs] = out
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(got[4].float()).all())
+    for bs in (16, 32, 128):
+        assert torch.equal(got[bs], got[4]), bs
+
+
 @pytest.mark.parametrize("dtype,head_dim,heads,kv_heads", [("bf16", 128, 16, 16), ("f32", 64, 4, 4),
                                                            ("bf16", 96, 6, 3), ("f32", 128, 2, 2)])
 def test_rope_kv_write_and_prefill_attention(dtype: str, head_dim: int, heads: int, kv_heads: int) -> None:
