@@ -552,9 +552,10 @@ CDB_DEVICE void load_floats(const float* p, float (&out)[N]) {
 
 constexpr int pow2_alignment(int bytes) { return bytes % 16 == 0 ? 16 : bytes % 8 == 0 ? 8 : 4; }
 
-template <typename T, int D>
+template <typename T, int D, int C>
 CDB_DEVICE void rotate_chunk(const RopeWriteParams& P, const T* base, const T* bias, int pos, int chunk, float* out) {
-  constexpr int C = D / 16;
+  constexpr int kLanes = D / C, kHalfLanes = kLanes / 2;
+  const int partner_chunk = chunk < kHalfLanes ? chunk + kHalfLanes : chunk - kHalfLanes;
   float own[C], partner[C];
   Vec<T, C> v;
   v.load(base + chunk * C);
@@ -562,7 +563,7 @@ CDB_DEVICE void rotate_chunk(const RopeWriteParams& P, const T* base, const T* b
   for (int i = 0; i < C; ++i) own[i] = v.get(i);
   const bool split_half = P.rope_style == 1;
   if (split_half) {
-    v.load(base + (chunk ^ 8) * C);
+    v.load(base + partner_chunk * C);
 #pragma unroll
     for (int i = 0; i < C; ++i) partner[i] = v.get(i);
   }
@@ -572,7 +573,7 @@ CDB_DEVICE void rotate_chunk(const RopeWriteParams& P, const T* base, const T* b
 #pragma unroll
     for (int i = 0; i < C; ++i) own[i] = Elem<T>::round(add_rn(own[i], bv.get(i)));
     if (split_half) {
-      bv.load(bias + (chunk ^ 8) * C);
+      bv.load(bias + partner_chunk * C);
 #pragma unroll
       for (int i = 0; i < C; ++i) partner[i] = Elem<T>::round(add_rn(partner[i], bv.get(i)));
     }
@@ -588,12 +589,12 @@ CDB_DEVICE void rotate_chunk(const RopeWriteParams& P, const T* base, const T* b
   const float* cr = P.rope_cos + (int64_t)pos * half;
   const float* sr = P.rope_sin + (int64_t)pos * half;
   if (split_half) {
-    // Elements d and d + D/2 share angle d mod D/2: the chunk's angles start at (chunk mod 8) * C.
+    // Elements d and d + D/2 share angle d mod D/2: the chunk's angles start at (chunk mod kHalfLanes) * C.
     float cs[C], sn[C];
-    const int f0 = (chunk & 7) * C;
+    const int f0 = (chunk < kHalfLanes ? chunk : chunk - kHalfLanes) * C;
     load_floats<C, pow2_alignment(C * 4)>(cr + f0, cs);
     load_floats<C, pow2_alignment(C * 4)>(sr + f0, sn);
-    const bool low = chunk < 8;
+    const bool low = chunk < kHalfLanes;
 #pragma unroll
     for (int i = 0; i < C; ++i) {
       const float rot = low ? -partner[i] : partner[i];
@@ -614,14 +615,16 @@ CDB_DEVICE void rotate_chunk(const RopeWriteParams& P, const T* base, const T* b
   }
 }
 
-template <typename T, int D>
+// D / C lanes per head, C elements each: sixteenths of a head, or 16-byte units (see
+// launch_rope_write). What bounds a long prompt is the traffic, half reads and half writes.
+template <typename T, int D, int C>
 __global__ void __launch_bounds__(kThreads) rope_kv_write_kernel(RopeWriteParams P) {
-  constexpr int C = D / 16;
-  const int lane = threadIdx.x & 63;
-  const int64_t group = blockIdx.x * (int64_t)(kThreads / 16) + (threadIdx.x >> 4);  // 16-lane group id
-  const int chunk = lane & 15;
+  constexpr int kLanes = D / C, kGroups = kThreads / kLanes;
+  const int local = threadIdx.x / kLanes;
+  const int64_t group = blockIdx.x * (int64_t)kGroups + local;
+  const int chunk = threadIdx.x - local * kLanes;
   const int64_t per_token = P.num_heads + P.num_kv_heads;
-  if (group >= P.tokens * per_token) return;
+  if (local >= kGroups || group >= P.tokens * per_token) return;
   const int64_t t = group / per_token;
   const int hh = (int)(group - t * per_token);
   const int pos = P.positions[t];
@@ -633,7 +636,7 @@ __global__ void __launch_bounds__(kThreads) rope_kv_write_kernel(RopeWriteParams
     T* dst = static_cast<T*>(P.q_out) + (t * P.num_heads + h) * D + chunk * C;
     Vec<T, C> ov;
     if (rope_ok) {
-      rotate_chunk<T, D>(P, src, P.q_bias ? static_cast<const T*>(P.q_bias) + (int64_t)h * D : nullptr, pos, chunk, o);
+      rotate_chunk<T, D, C>(P, src, P.q_bias ? static_cast<const T*>(P.q_bias) + (int64_t)h * D : nullptr, pos, chunk, o);
 #pragma unroll
       for (int i = 0; i < C; ++i) ov.set(i, o[i]);
     } else {
@@ -651,7 +654,7 @@ __global__ void __launch_bounds__(kThreads) rope_kv_write_kernel(RopeWriteParams
   const int64_t row = P.rows[t];
   if (row < 0 || row >= P.pool_rows || !rope_ok) return;
   float o[C];
-  rotate_chunk<T, D>(P, static_cast<const T*>(P.k) + t * P.kv_stride + (int64_t)kvh * D,
+  rotate_chunk<T, D, C>(P, static_cast<const T*>(P.k) + t * P.kv_stride + (int64_t)kvh * D,
                      P.k_bias ? static_cast<const T*>(P.k_bias) + (int64_t)kvh * D : nullptr, pos, chunk, o);
   const int64_t off = (int64_t)P.layer * P.layer_stride + (row * P.num_kv_heads + kvh) * D + chunk * C;
   Vec<T, C> kw;
@@ -687,11 +690,42 @@ int launch_norm(const NormParams& P, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
 }
 
+template <typename T, int D, int C>
+int launch_rope_write_chunks(const RopeWriteParams& P, hipStream_t s) {
+  constexpr int kGroups = kThreads / (D / C);
+  const int64_t blocks = (P.tokens * (P.num_heads + P.num_kv_heads) + kGroups - 1) / kGroups;
+  if (blocks > 0x7fffffff) return CDB_ERR_SHAPE;
+  hipLaunchKernelGGL((rope_kv_write_kernel<T, D, C>), dim3((unsigned)blocks), dim3(kThreads), 0, s, P);
+  return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
+}
+
+// Sixteenths of a head are 8 or 16 bytes for bf16 heads of 64 and 128 and float heads of 64: one
+// access per lane and row part. The other heads (12 bytes, three 4-byte accesses; 24 and 32
+// bytes, several with gaps between the lanes) take 16-byte units where everything is aligned to
+// them: 55 heads x 96 in bf16, 4000 tokens, 70 -> 62 us and 512 or fewer the same (10 us); 16 heads
+// x 128 in float, 4000 tokens, 54 -> 47 us, 100 tokens 3.6 -> 3.3. (8-byte sixteenths in 16-byte
+// units were slower: 12 + 4 heads x 64, 2000 tokens, 5.0 -> 7.2 us.) The halves of a head
+// may then lie in different waves, so what is read must not be what is written.
 template <typename T, int D>
 int launch_rope_write(const RopeWriteParams& P, hipStream_t s) {
-  const int64_t groups = P.tokens * (P.num_heads + P.num_kv_heads);
-  hipLaunchKernelGGL((rope_kv_write_kernel<T, D>), dim3(grid_for(groups, kThreads / 16)), dim3(kThreads), 0, s, P);
-  return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
+  constexpr int64_t kElem = sizeof(T);
+  if constexpr (D / 16 * kElem != 8 && D / 16 * kElem != 16) {
+    const uintptr_t at = (uintptr_t)P.q | (uintptr_t)P.k | (uintptr_t)P.v | (uintptr_t)P.q_out | (uintptr_t)P.k_pool |
+                         (uintptr_t)P.v_pool | (uintptr_t)P.rope_cos | (uintptr_t)P.rope_sin | (uintptr_t)P.q_bias |
+                         (uintptr_t)P.k_bias;
+    const int64_t strides = (P.q_stride | P.kv_stride | P.layer_stride) * kElem;
+    const int64_t pool_bytes = P.pool_rows * P.num_kv_heads * D * kElem, pool_at = P.layer * P.layer_stride * kElem;
+    auto overlap = [&](const void* src, int64_t stride, int heads, const void* dst, int64_t dst_at, int64_t bytes) {
+      const uintptr_t s0 = (uintptr_t)src, s1 = s0 + ((P.tokens - 1) * stride + (int64_t)heads * D) * kElem;
+      const uintptr_t d0 = (uintptr_t)dst + dst_at, d1 = d0 + bytes;
+      return s0 < d1 && d0 < s1;
+    };
+    const bool apart = !overlap(P.q, P.q_stride, P.num_heads, P.q_out, 0, P.tokens * P.num_heads * D * kElem) &&
+                       !overlap(P.k, P.kv_stride, P.num_kv_heads, P.k_pool, pool_at, pool_bytes) &&
+                       !overlap(P.v, P.kv_stride, P.num_kv_heads, P.v_pool, pool_at, pool_bytes);
+    if (apart && ((at | strides) & 15) == 0) return launch_rope_write_chunks<T, D, 16 / kElem>(P, s);
+  }
+  return launch_rope_write_chunks<T, D, D / 16>(P, s);
 }
 
 }  // namespace

@@ -311,6 +311,41 @@ def test_exit_kv_copy_bit_exact() -> None:
     np.testing.assert_array_equal(host(pt), want)
 
 
+@pytest.mark.parametrize("dtype,head_dim", [("bf16", 96), ("f32", 96), ("f32", 128)])
+@pytest.mark.parametrize("style", [0, 1, 2])
+def test_rope_kv_write_in_16_byte_units(dtype: str, head_dim: int, style: int) -> None:
+    """Heads whose sixteenths are no 16-byte access take 16-byte units where all is aligned: the bits
+    of the general form, which the same rows 8 bytes off alignment and queries rotated in place
+    take, with head counts around a workgroup's and out-of-range rows and positions."""
+
+    from continuous_depth_batching_amd import ops
+
+    tokens, heads, kv_heads, bs = 5, 23, 3, 4
+    torch.manual_seed(head_dim + style)
+    dt, off = DT[dtype], 8 // (2 if dtype == "bf16" else 4)
+    mk = lambda h: torch.randn(tokens, h, head_dim, device="cuda").to(dt)
+    q, k, v = mk(heads), mk(kv_heads), mk(kv_heads)
+    qb, kb = torch.randn(heads * head_dim, device="cuda").to(dt), torch.randn(kv_heads * head_dim, device="cuda").to(dt)
+    cos, sin = torch.randn(9, head_dim // 2, device="cuda"), torch.randn(9, head_dim // 2, device="cuda")
+    rows = torch.tensor([3, 8, -1, 0, 5], device="cuda")
+    pos = torch.tensor([8, 0, 4, 9, 2], dtype=torch.int32, device="cuda")
+
+    def shifted(t: torch.Tensor) -> torch.Tensor:
+        flat = torch.empty(t.numel() + off, dtype=t.dtype, device="cuda")[off:]
+        return flat.copy_(t.flatten()).view(t.shape)
+
+    outs = []
+    for form in ("units", "misaligned", "in place"):
+        qi, ki, vi = (shifted(t) if form == "misaligned" else t.clone() for t in (q, k, v))
+        pool = torch.zeros(2, 2, 12, kv_heads, head_dim, dtype=dt, device="cuda")
+        qo = qi if form == "in place" else torch.empty_like(q)
+        ops.rope_kv_write_raw(qi, ki, vi, qo, ops.KVPoolView(pool, bs), 1, rows, pos, cos, sin, style, qb, kb)
+        outs.append((torch.nan_to_num(qo.float(), nan=1e30), pool))
+    for qo, pool in outs[1:]:
+        assert torch.equal(qo, outs[0][0]) and torch.equal(pool, outs[0][1])
+    assert bool((outs[0][1][1, 0, 8] != 0).any()) and bool((outs[0][0][3] == 1e30).all()) == (style != 0)
+
+
 @pytest.mark.parametrize("head_dim", [64, 96, 128])
 @pytest.mark.parametrize("split", [False, True])
 def test_prefill_attention_does_not_depend_on_the_page_size(head_dim: int, split: bool) -> None:
