@@ -311,6 +311,32 @@ def test_exit_kv_copy_bit_exact() -> None:
     np.testing.assert_array_equal(host(pt), want)
 
 
+@pytest.mark.parametrize("heads,head_dim,layers,slots,n", [(55, 96, 1, 3, 2), (3, 64, 2, 33, 1), (3, 64, 2, 33, 70),
+                                                           (1, 8, 1, 2, 5)])
+def test_exit_kv_copy_over_targets_and_row_pieces(heads: int, head_dim: int, layers: int, slots: int, n: int) -> None:
+    """Rows longer and shorter than one workgroup's 4 KiB, with each workgroup storing one target or
+    several: every deeper slot gets the exit slot's bits and nothing else changes, for exits at
+    every slot, at the last and at none, and for rows that the pool does not have."""
+
+    from continuous_depth_batching_amd import ops
+
+    torch.manual_seed(n)
+    bs, rows_n = 4, 80
+    pool = torch.randn(1 + layers * slots, 2, rows_n, heads, head_dim, device="cuda").bfloat16()
+    rows = torch.randperm(rows_n)[:n]
+    exits = torch.arange(n) % (slots + 1) - 1
+    if n > 2:
+        rows[1] = rows_n
+    want = pool.cpu()
+    for row, e in zip(rows.tolist(), exits.tolist()):
+        if 0 <= e and row < rows_n:
+            for s in range(e + 1, slots):
+                want[1 + s * layers:1 + (s + 1) * layers, :, row] = want[1 + e * layers:1 + (e + 1) * layers, :, row]
+    ops.exit_kv_copy_raw(ops.KVPoolView(pool, bs), rows.cuda(), exits.int().cuda(), n, layer_base=1,
+                         core_layers=layers, num_slots=slots)
+    assert torch.equal(pool.cpu(), want)
+
+
 @pytest.mark.parametrize("dtype,head_dim", [("bf16", 96), ("f32", 96), ("f32", 128)])
 @pytest.mark.parametrize("style", [0, 1, 2])
 def test_rope_kv_write_in_16_byte_units(dtype: str, head_dim: int, style: int) -> None:
