@@ -65,9 +65,8 @@ def parse_args() -> argparse.Namespace:
     p.add_argument("--cpu-sample-tokens", type=int, default=160)
     p.add_argument("--attention-iters", type=int, default=20)
     p.add_argument("--attention-rows", type=int, default=256,
-                   help="decode-attention: time the first N rows of the 256-row shape (up to 256 rows of "
-                        "128-wide heads run the deep form, which merges in the decode kernel); the bench "
-                        "line keeps 256")
+                   help="decode-attention: time the first N rows of the 256-row shape (128-wide heads run the "
+                        "deep form, which merges in the decode kernel); the bench line keeps 256")
     return p.parse_args()
 
 
@@ -447,11 +446,10 @@ def time_companion_kernels(rows: int = 1024, hidden: int = 2048, prefill_tokens:
 
 def decode_kernels(rows: int) -> str:
     """The kernels one attend call runs at ``rows`` rows of 16-token pages (the decode library's
-    form choice at 128-wide heads: the deep form, which merges in the decode kernel, up to 256 rows)."""
+    form choice at 128-wide heads: the deep form, which merges in the decode kernel, with three K/V
+    buffers per wave up to 256 rows and two above)."""
 
-    if rows <= 256:
-        return "cdb::paged_decode_deep_kernel<bf16,128> (merge in the kernel)"
-    return "cdb::paged_decode_fast_kernel<bf16,128> + decode_merge_kernel"
+    return f"cdb::paged_decode_deep_kernel<bf16,128,{3 if rows <= 256 else 2} buffers> (merge in the kernel)"
 
 
 TRAFFIC_RECORD = "profiles/decode_attention_c2_256rows_traffic.json"

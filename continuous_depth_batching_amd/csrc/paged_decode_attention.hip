@@ -23,15 +23,16 @@
 //   * one decode kernel. A work item is (chunk, query head) and belongs to one
 //     wave of a persistent grid, which takes items in the plan's order, so the
 //     longest items go first and every wave ends on short ones.
-//     - paged_decode_fast_kernel (16-token pages, 8-page chunks: the engine's
-//       shape; more than kDeepRowsOf<D> rows): while a wave streams one item it
-//       already holds the next item's descriptor and loads its query and new
-//       token, and the next item's first K/V step is issued into the buffer the
-//       current item's last step frees; the launch's tail goes to whichever
-//       wave asks first, from its XCD's queue.
-//     - paged_decode_deep_kernel (the same shape, at most kDeepRowsOf<D> rows): each
-//       wave keeps three K/V steps in flight, and the wave that stores a row's
-//       last chunk merges the row (arrival counters, agent-coherent partials).
+//     - paged_decode_deep_kernel (16-token pages, 8-page chunks: the engine's
+//       shape): each wave keeps one or two K/V steps in flight besides the one it
+//       computes, and the wave that stores a row's last chunk merges the row
+//       (arrival counters, agent-coherent partials).
+//     - paged_decode_fast_kernel (the same shape, more than kPersistentRows rows of
+//       64-wide heads): while a wave streams one item it already holds the next
+//       item's descriptor and loads its query and new token, and the next item's
+//       first K/V step is issued into the buffer the current item's last step
+//       frees; the launch's tail goes to whichever wave asks first, from its XCD's
+//       queue.
 //     - paged_decode_kernel: any page size and chunk length.
 //   * decode_merge_kernel (after the fast and general forms) combines the
 //     partials of rows with several chunks, in chunk order, and fills the
@@ -893,7 +894,11 @@ CDB_DEVICE FastItem make_fast_item(const DecodeParams& P, const RawFastDesc& r, 
 // reads page 0 of the layer (any valid address) and every token of a masked
 // page or at/after t_end gets zero weight. The pages are read once per layer,
 // so the loads carry the nontemporal hint (the deep form measured 4-7% faster
-// with it, the persistent form 1-2%, and the headline decode run 3%).
+// with it, the persistent form 1-2%, and the headline decode run 3%). Not so for
+// 96-wide heads, whose bf16 rows of 192 bytes share a 128-byte line with the next
+// head's: cached, the waves of a workgroup (consecutive heads) find the other half
+// in L2 (fetched bytes 1.25x -> 1.14x of those needed; 128 rows of 55 heads, two
+// layers: 616 -> 580 us; in float 1079 -> 991).
 template <typename T, int D>
 CDB_DEVICE void load_fast_step(const DecodeParams& P, const FastItem& f, int s, const uint32_t (&lane_off)[4],
                                int slot, Vec<T, D / 16> (&kv)[4], Vec<T, D / 16> (&vv)[4], bool (&valid)[4]) {
@@ -905,8 +910,13 @@ CDB_DEVICE void load_fast_step(const DecodeParams& P, const FastItem& f, int s, 
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     valid[u] = blk >= 0 && t0 + 4 * u + slot < f.it.t_end;
-    kv[u].load_nt(reinterpret_cast<const T*>(kp + lane_off[u]));
-    vv[u].load_nt(reinterpret_cast<const T*>(vp + lane_off[u]));
+    if constexpr (D == 96) {
+      kv[u].load(reinterpret_cast<const T*>(kp + lane_off[u]));
+      vv[u].load(reinterpret_cast<const T*>(vp + lane_off[u]));
+    } else {
+      kv[u].load_nt(reinterpret_cast<const T*>(kp + lane_off[u]));
+      vv[u].load_nt(reinterpret_cast<const T*>(vp + lane_off[u]));
+    }
   }
 }
 
@@ -1120,18 +1130,21 @@ __global__ void __launch_bounds__(256, 3) paged_decode_fast_kernel(DecodeParams 
   }
 }
 
-// The fast form for launches of up to kDeepRowsOf<D> rows: such a launch gives a
-// wave a few items, so latency matters more than occupancy. Each wave keeps kDeepSteps - 1 steps of K/V in
-// flight (four register buffers, 2 waves per SIMD) instead of one, and takes
-// its items without cross-item prefetch. A chunk is computed exactly as in
-// paged_decode_fast_kernel (same steps in the same order, same masking, same
-// new-token and slot merge), so a row's result does not depend on the form.
-// The limit is where the deep form stops measuring faster than the persistent
-// one: 256 rows for 128-wide heads (with the nontemporal K/V loads, 4-8% faster
-// from 128 to 256 rows, no merge launch; 120 rows before them), 120 rows for the
-// other head sizes, where it was measured with cached loads.
+// The deep form: each wave keeps kBuffers - 1 steps of K/V in flight and takes its items
+// without cross-item prefetch, and the last wave to store a row's chunk merges the row. A chunk
+// is computed exactly as in paged_decode_fast_kernel (same steps in the same order, same masking,
+// same new-token and slot merge), so a row's result does not depend on the form.
+// Up to kDeepRowsOf<D> rows a wave has a few items and latency counts: three buffers (16 rows of 12
+// heads x 64, two layers with the plan: 38.1 us against 40.4 with two; 256 rows of 16 x 128: 363
+// against 374, and 387 with four). Above, two leave room for more waves (512 rows of 16 x 128: 431
+// us against 448 with three; 1024: 406 against 420).
 template <int D> constexpr int kDeepRowsOf = D == 128 ? 256 : 120;
-constexpr int kDeepSteps = 4;
+// The persistent form stays where its prefetch across items still pays: many rows of 64-wide
+// heads, whose items are half as long (12 heads, two layers: 174 us against 171 with the deep form
+// at 256 rows, 309 against 327 at 512, 368 against 389 at 1000). At 128 wide it took 461 us
+// against 431 at 512 rows and 433 against 406 at 1024; at 55 heads x 96 606 against 580 at 128
+// rows; in float at 16 x 128, where it spills, 6.5 ms against 3.1 at 300 rows of 1500-2000 tokens.
+constexpr int kPersistentRows = 256;
 
 template <typename T, int D, bool kCoherent = false>
 CDB_DEVICE void merge_chunks(const float* part, int64_t stride, int nsplit, int lane, T* out_row);
@@ -1215,7 +1228,7 @@ CDB_DEVICE void fill_chunkless_rows(const DecodeParams& P, int wave_id, int nwav
   }
 }
 
-template <typename T, int D, int R>
+template <typename T, int D, int R, int kBuffers>
 __global__ void __launch_bounds__(256, 2) paged_decode_deep_kernel(DecodeParams P) {
   constexpr int C = Layout<D>::kChunk;
   const int lane = threadIdx.x & 63;
@@ -1241,10 +1254,10 @@ __global__ void __launch_bounds__(256, 2) paged_decode_deep_kernel(DecodeParams 
     issue_pending<T, D, R>(P, c, chunk, pend);
     Angles<D> ang;
     load_angles<D, R>(P, c.p, chunk, ang);
-    Vec<T, C> kbuf[kDeepSteps][4], vbuf[kDeepSteps][4];
-    bool vl[kDeepSteps][4];
+    Vec<T, C> kbuf[kBuffers][4], vbuf[kBuffers][4];
+    bool vl[kBuffers][4];
 #pragma unroll
-    for (int st = 0; st < kDeepSteps - 1; ++st) load_fast_step<T, D>(P, cur, st, lane_off, slot, kbuf[st], vbuf[st], vl[st]);
+    for (int st = 0; st < kBuffers - 1; ++st) load_fast_step<T, D>(P, cur, st, lane_off, slot, kbuf[st], vbuf[st], vl[st]);
 
     QueryReg<T, D> q;
     Vec<T, C> kn, vn;
@@ -1269,11 +1282,11 @@ __global__ void __launch_bounds__(256, 2) paged_decode_deep_kernel(DecodeParams 
 #pragma unroll
     for (int st = 0; st < kChunkPagesFast; ++st) {
       if (st >= steps) break;
-      const int ahead = st + kDeepSteps - 1;
+      const int ahead = st + kBuffers - 1;
       if (ahead < kChunkPagesFast)
-        load_fast_step<T, D>(P, cur, ahead, lane_off, slot, kbuf[ahead % kDeepSteps], vbuf[ahead % kDeepSteps],
-                             vl[ahead % kDeepSteps]);
-      attend_step<T, D>(q, P.scale_log2, kbuf[st % kDeepSteps], vbuf[st % kDeepSteps], vl[st % kDeepSteps], m, l,
+        load_fast_step<T, D>(P, cur, ahead, lane_off, slot, kbuf[ahead % kBuffers], vbuf[ahead % kBuffers],
+                             vl[ahead % kBuffers]);
+      attend_step<T, D>(q, P.scale_log2, kbuf[st % kBuffers], vbuf[st % kBuffers], vl[st % kBuffers], m, l,
                         acc);
     }
 
@@ -1494,15 +1507,21 @@ int launch_decode(const DecodeParams& P, int stages, int num_cus, hipStream_t st
     if (hipGetLastError() != hipSuccess) return CDB_ERR_HIP;
   }
   if (!(stages & CDB_DECODE_STAGE_ATTEND)) return CDB_OK;
-  const bool deep = fast_form(P) && P.num_rows <= kDeepRowsOf<D>;
-  const int rc = !fast_form(P) ? launch_persistent(paged_decode_kernel<T, D, R>, P, num_cus, stream)
-                 : deep        ? launch_persistent(paged_decode_deep_kernel<T, D, R>, P, num_cus, stream)
-                               : launch_persistent(paged_decode_fast_kernel<T, D, R>, P, num_cus, stream);
+  DecodeKernel kernel = paged_decode_kernel<T, D, R>;
+  bool merged = false;
+  if (fast_form(P)) {
+    merged = D != 64 || P.num_rows <= kPersistentRows;
+    kernel = P.num_rows <= kDeepRowsOf<D> ? paged_decode_deep_kernel<T, D, R, 3> : paged_decode_deep_kernel<T, D, R, 2>;
+    if constexpr (D == 64) {
+      if (!merged) kernel = paged_decode_fast_kernel<T, D, R>;
+    }
+  }
+  const int rc = launch_persistent(kernel, P, num_cus, stream);
   if (rc != CDB_OK) return rc;
   // A deep launch has merged and filled every row itself (against the merge launch, same box, per
   // layer, with the partials' 8-byte coherent stores: 0.1-0.5 us faster from 1 to 16 rows, 1-2 us
   // from 24 to 120 rows); the others end with the merge launch.
-  if (deep) return CDB_OK;
+  if (merged) return CDB_OK;
   const int64_t waves = (int64_t)P.num_rows * P.num_heads;
   hipLaunchKernelGGL((decode_merge_kernel<T, D>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, P);
   return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;

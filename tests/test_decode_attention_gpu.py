@@ -207,9 +207,8 @@ def _attend(case, d, ws, rows, cache_layer0=0, stages=None):
 def test_row_output_is_bit_identical_in_any_batch_composition() -> None:
     # A row's chunks and their merge order depend only on the row: alone, inside the
     # full batch, or inside a shuffled half of it, its output is the same to the bit.
-    # 272 rows run the persistent fast form and the merge launch (more than the deep form's
-    # 256 rows at 128-wide heads); 136 rows, 30 rows and single rows the deep form, which
-    # merges in the decode kernel.
+    # 272 rows run the deep form with two buffers (more than 256 rows at 128-wide heads);
+    # 136 rows, 30 rows and single rows the one with three.
     case = make_case(seed=31, num_rows=272, num_heads=16, num_kv_heads=16, head_dim=128, max_context=1500,
                      rope_style=1, dtype="bf16", padding_rows=3)
     d, ws = _device_case(case)
@@ -228,7 +227,7 @@ def test_row_output_is_bit_identical_in_any_batch_composition() -> None:
 
 def test_huginn_shape_row_output_is_bit_identical_in_any_batch_composition() -> None:
     # The same at Huginn-0125's attention shape (55 heads x 96, interleaved RoPE with q/k
-    # bias): 150 rows run the persistent fast form, 75 rows and single rows the deep form.
+    # bias): 150 rows run the deep form with two buffers, 75 rows and single rows with three.
     case = make_case(seed=34, num_rows=150, num_heads=55, num_kv_heads=55, head_dim=96, max_context=700,
                      rope_style=2, dtype="bf16", padding_rows=2, qk_bias=True)
     d, ws = _device_case(case)
@@ -243,6 +242,22 @@ def test_huginn_shape_row_output_is_bit_identical_in_any_batch_composition() -> 
         assert torch.equal(_attend(case, d, ws, [r])[0], full[r])
 
 
+@pytest.mark.parametrize("dtype,heads,head_dim,rows", [("bf16", 3, 64, 121), ("bf16", 3, 64, 257), ("f32", 3, 64, 257),
+                                                       ("bf16", 5, 96, 121), ("f32", 5, 96, 121),
+                                                       ("bf16", 2, 128, 257), ("f32", 2, 128, 257)])
+def test_forms_agree_where_the_row_count_changes_them(dtype: str, heads: int, head_dim: int, rows: int) -> None:
+    """One row more than a form's limit, at the limit and a few rows: the same bits in each."""
+
+    case = make_case(seed=rows + head_dim, num_rows=rows, num_heads=heads, num_kv_heads=heads, head_dim=head_dim,
+                     max_context=400, rope_style=1, dtype=dtype, padding_rows=2)
+    d, ws = _device_case(case)
+    full = _attend(case, d, ws, list(range(rows)))
+    less = _attend(case, d, ws, list(range(1, rows)))
+    few = _attend(case, d, ws, list(range(20)))
+    torch.cuda.synchronize()
+    assert torch.equal(less, full[1:]) and torch.equal(few, full[:20])
+
+
 FAST_FORM_SHAPES = {
     # name: (dtype, heads, kv_heads, head_dim, rope_style, qk_bias)
     "f32-mha-16x128": ("f32", 16, 16, 128, 1, False),
@@ -254,10 +269,9 @@ FAST_FORM_SHAPES = {
 @pytest.mark.parametrize("rows", [96, 272])
 @pytest.mark.parametrize("shape", sorted(FAST_FORM_SHAPES))
 def test_wide_launches_against_the_oracle(shape: str, rows: int) -> None:
-    """Against the float64 oracle: 272 rows (more than the deep form's limit, 256 rows at 128-wide
-    heads and 120 at the others, so the persistent fast form with its XCD tail queues, cross-item
-    prefetch, LDS stash and merge launch runs) and 96 rows (the deep form, whose last-arriving waves
-    merge each row's chunks in the decode kernel). Both
+    """Against the float64 oracle: 272 rows (the deep form with two buffers, and at 64-wide heads the
+    persistent form with its XCD tail queues, cross-item prefetch, LDS stash and merge launch) and 96
+    rows (the deep form with three; its last-arriving waves merge each row's chunks). Both
     with padding rows, multi-chunk rows, one row past its block table and one row at a cache layer
     outside the pool: those two get NaN and write nothing, every other row is within the bar and
     its appended K/V row is bit-identical to the oracle's. Two calls run on one workspace, so the
