@@ -91,9 +91,9 @@ CDB_DEVICE f32x4_t sum_slots(const f32x4_t (&red)[SLOTS][NT][MT][kWave], int til
 // of y, store each row's greedy-argmax candidate of every 16-column tile (the
 // largest bf16-rounded output and its first column, torch.argmax order), for
 // linear_argmax_merge_kernel.
-template <int MT, int NB, int S, int SLOTS, int MAXT, bool ARGMAX = false>
+template <int MT, int NB, int S, int SLOTS, bool GATED, int MAXT, bool ARGMAX = false>
 __global__ void __launch_bounds__(MAXT) linear_kernel(LinearParams p) {
-  constexpr int NT = NB;
+  constexpr int NT = GATED ? 2 * NB : NB;  // W row tiles: gate tiles, then up tiles
   __shared__ f32x4_t red[SLOTS][NT][MT][kWave];
 
   const int lane = threadIdx.x & (kWave - 1);
@@ -107,7 +107,10 @@ __global__ void __launch_bounds__(MAXT) linear_kernel(LinearParams p) {
   const int total = p.K / 32;
   const bf16_t* wrow[NT];
 #pragma unroll
-  for (int j = 0; j < NB; ++j) wrow[j] = p.w + ((int64_t)(n0 / 16 + j) * total) * 512 + 8 * lane;
+  for (int j = 0; j < NB; ++j) {
+    wrow[j] = p.w + ((int64_t)(n0 / 16 + j) * total) * 512 + 8 * lane;
+    if constexpr (GATED) wrow[NB + j] = p.w + ((int64_t)((p.N + n0) / 16 + j) * total) * 512 + 8 * lane;
+  }
   const bf16_t* xrow[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) xrow[mt] = p.x + (int64_t)min(mt * 16 + r, p.M - 1) * p.ldx + 8 * g;
@@ -212,9 +215,19 @@ __global__ void __launch_bounds__(MAXT) linear_kernel(LinearParams p) {
     const int m = mt * 16 + (l & 15);
     if (m < p.M) {
       const f32x4_t v = sum_slots(red, j, mt, l, slots);
+      f32x4_t u = {};
+      if constexpr (GATED) u = sum_slots(red, NB + j, mt, l, slots);
       Vec<bf16_t, 4> o;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o.set(i, v[i]);
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (GATED) {
+          const float gate = round_bf16(v[i]);
+          const float act = silu_bf16(gate);
+          o.set(i, act * round_bf16(u[i]));
+        } else {
+          o.set(i, v[i]);
+        }
+      }
       o.store(p.y + (int64_t)m * p.ldy + n0 + 16 * j + 4 * (l >> 4));
     }
   }
@@ -689,8 +702,8 @@ __global__ void __launch_bounds__(kArgmaxMergeThreads) linear_argmax_merge_kerne
 // Launch shape of one instantiation: threads per workgroup are capped so the
 // accumulators and a batch of loads fit without spilling, and the LDS partial
 // tiles (SLOTS x NT x MT x 1 KiB) stay within 64 KiB.
-template <int MT, int NB, int S> struct LinearShape {
-  static constexpr int kNT = NB;
+template <int MT, int NB, int S, bool GATED> struct LinearShape {
+  static constexpr int kNT = GATED ? 2 * NB : NB;
   static constexpr int kRegs = 4 * (kNT * S + MT * S + kNT * MT);
   static constexpr int kThreads = kRegs <= 96 ? 1024 : 512;
   static constexpr int kSlots = 64 / (kNT * MT) < 8 ? 64 / (kNT * MT) : 8;
@@ -705,14 +718,14 @@ inline int linear_steps_per_wave(int32_t in_features, int batch, int max_waves) 
   return (per_wave + batch - 1) / batch * batch;
 }
 
-template <int MT, int NB, int S, bool ARGMAX = false>
+template <int MT, int NB, int S, bool GATED, bool ARGMAX = false>
 int launch_linear(LinearParams prm, hipStream_t stream, int max_waves = kLinearMaxWaves) {
-  using Shape = LinearShape<MT, NB, S>;
+  using Shape = LinearShape<MT, NB, S, GATED>;
   if (prm.N % (16 * NB)) return CDB_ERR_SHAPE;
   const int waves_cap = max_waves < Shape::kMaxWaves ? max_waves : Shape::kMaxWaves;
   prm.steps_per_wave = linear_steps_per_wave(prm.K, S, waves_cap);
   const int nwaves = (prm.K / 32 + prm.steps_per_wave - 1) / prm.steps_per_wave;
-  hipLaunchKernelGGL((linear_kernel<MT, NB, S, Shape::kSlots, Shape::kThreads, ARGMAX>),
+  hipLaunchKernelGGL((linear_kernel<MT, NB, S, Shape::kSlots, GATED, Shape::kThreads, ARGMAX>),
                      dim3(prm.N / (16 * NB)), dim3(nwaves * kWave), 0, stream, prm);
   return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
 }
@@ -729,9 +742,14 @@ namespace {
 // one, so N = 2048 still spreads over 128 CUs. Batches of 4 steps (2 at four row
 // tiles, for registers); 8 waves per workgroup for one row tile, 4 above.
 template <int MT, int S>
-int dispatch_rows(const LinearParams& prm, int max_waves, hipStream_t stream) {
-  return prm.N >= 4096 && prm.N % 32 == 0 ? launch_linear<MT, 2, S>(prm, stream, max_waves)
-                                          : launch_linear<MT, 1, S>(prm, stream, max_waves);
+int dispatch_rows(const LinearParams& prm, bool gated, int max_waves, hipStream_t stream) {
+  const bool wide = prm.N >= 4096 && prm.N % 32 == 0;
+  if (wide) {
+    return gated ? launch_linear<MT, 2, S, true>(prm, stream, max_waves)
+                 : launch_linear<MT, 2, S, false>(prm, stream, max_waves);
+  }
+  return gated ? launch_linear<MT, 1, S, true>(prm, stream, max_waves)
+               : launch_linear<MT, 1, S, false>(prm, stream, max_waves);
 }
 
 enum class StreamMode { kPlain, kGated, kParts };
@@ -848,20 +866,15 @@ int dispatch_parts(const LinearParams& prm, int splits, hipStream_t stream) {
   return dispatch_stream(prm, StreamMode::kParts, splits, stream);
 }
 
-// The row kernel's share of up to 32 rows: plain projections of fewer than 8192 columns up to
-// 16 rows (2048 -> 6144 at 1 / 13 rows 6.4 / 7.1 us against 7.9 / 8.0 streamed, 10560 -> 5280 at
-// 16 rows 26 against 31; from 5280 -> 15840 on the streaming form wins, 29.1 against 31.8 at 16
-// rows), and the LM heads, whose logits then equal those of the argmax form bit for bit.
-// Gated projections stream at every batch: 2048 -> 2 x 5632 at 16 rows 11.4 -> 10.0 us,
-// 5280 -> 2 x 17920 72 -> 61 us.
-bool use_row_kernel(const LinearParams& prm, bool gated) {
-  return !gated && (prm.M <= 16 ? prm.N < 8192 || prm.N > 16384 : prm.M <= 32 && prm.N > 16384);
-}
-
+// The row kernel keeps every shape of at most 64 rows that wide_path does not name. The streaming
+// form is faster for some of them (2048 -> 2 x 5632 gated at 16 rows 11.4 -> 10.0 us, 5280 -> 2 x
+// 17920 72 -> 61), but it adds all of K in one accumulator where the row kernel adds four or eight
+// partial sums, and its rounding error against 64 bits must not grow.
 int dispatch_linear(const LinearParams& prm, bool gated, hipStream_t stream) {
-  if (use_row_kernel(prm, gated))
-    return prm.M <= 16 ? dispatch_rows<1, 4>(prm, 8, stream) : dispatch_rows<2, 4>(prm, 4, stream);
-  return dispatch_stream(prm, gated ? StreamMode::kGated : StreamMode::kPlain, 1, stream);
+  if (wide_path(prm)) return dispatch_stream(prm, gated ? StreamMode::kGated : StreamMode::kPlain, 1, stream);
+  if (prm.M <= 16) return dispatch_rows<1, 4>(prm, gated, 8, stream);
+  if (prm.M <= 32) return dispatch_rows<2, 4>(prm, gated, 4, stream);
+  return dispatch_rows<4, 2>(prm, gated, 4, stream);
 }
 
 }  // namespace
@@ -972,11 +985,11 @@ extern "C" int cdb_linear_argmax(const void* x, int64_t ldx, const void* w_packe
   const bool two = out_features >= 4096 && out_features % 32 == 0;
   int rc;
   if (rows <= 16)
-    rc = two ? launch_linear<1, 2, 4, true>(prm, stream, 8) : launch_linear<1, 1, 4, true>(prm, stream, 8);
+    rc = two ? launch_linear<1, 2, 4, false, true>(prm, stream, 8) : launch_linear<1, 1, 4, false, true>(prm, stream, 8);
   else if (rows <= 32)
-    rc = two ? launch_linear<2, 2, 4, true>(prm, stream, 4) : launch_linear<2, 1, 4, true>(prm, stream, 4);
+    rc = two ? launch_linear<2, 2, 4, false, true>(prm, stream, 4) : launch_linear<2, 1, 4, false, true>(prm, stream, 4);
   else
-    rc = two ? launch_linear<4, 2, 2, true>(prm, stream, 4) : launch_linear<4, 1, 2, true>(prm, stream, 4);
+    rc = two ? launch_linear<4, 2, 2, false, true>(prm, stream, 4) : launch_linear<4, 1, 2, false, true>(prm, stream, 4);
   if (rc != CDB_OK) return rc;
   ArgmaxEmbed emb{static_cast<const bf16_t*>(embed), static_cast<bf16_t*>(bank), bank_slots, out_features,
                   bank_rows, width};
