@@ -397,14 +397,14 @@ def linear_raw(x: torch.Tensor, packed: torch.Tensor, out: torch.Tensor, *, gate
                "cdb_linear")
 
 
-# Batches up to this many rows run the wide-tile kernel when the shape qualifies.
+# Batches up to this many rows run the streaming kernel when the shape qualifies.
 LINEAR_WIDE_MAX_ROWS = 256
 
 
 def linear_prefers_kernel(rows: int, out_features: int, gated: bool, in_features: int = 0) -> bool:
     """Whether cdb_linear beats torch.mm for this batch (measured on cold weights): always
     up to 32 rows; up to 64 for the gated MLP projection (its fused SiLU saves a pass) and
-    for outputs of 4096 to 16384 columns; and up to 256 rows on the wide-tile kernel for
+    for outputs of 4096 to 16384 columns; and up to 256 rows on the streaming kernel for
     2048-wide inputs with such outputs (a multiple of 128 columns), and up to 128 rows for
     5280-wide inputs with such outputs or a gated one. The LM heads (49152 and 65536
     columns) above 32 rows are faster on hipBLASLt, as are O and down projections."""
@@ -414,7 +414,7 @@ def linear_prefers_kernel(rows: int, out_features: int, gated: bool, in_features
     mid = 4096 <= out_features <= 16384
     if rows <= LINEAR_MAX_ROWS and (gated or mid):
         return True
-    if in_features == 5280:  # Huginn QKV and gate/up on the wide-tile kernel up to 128 rows
+    if in_features == 5280:  # Huginn QKV and gate/up on the streaming kernel up to 128 rows
         return rows <= 128 and (gated or mid)
     return rows <= LINEAR_WIDE_MAX_ROWS and mid and out_features % 128 == 0 and in_features == 2048
 

@@ -253,13 +253,14 @@ def test_wide_tile_forms_give_a_row_the_same_bits_in_any_batch() -> None:
     assert ((gated[256].float() - ref).abs() <= 2 * _bf16_ulp(ref) + 1e-3).float().mean().item() >= 0.99
 
 
-@pytest.mark.parametrize("rows", [17, 33, 64])
-@pytest.mark.parametrize("k", [32, 96, 256, 288, 512, 544])
-@pytest.mark.parametrize("n", [16, 112])
+@pytest.mark.parametrize("rows,k,n", [(17, 544, 112), (64, 96, 16), (33, 2048, 4096), (65, 2048, 4224),
+                                      (129, 2048, 4096), (241, 2048, 4224), (256, 2048, 4096), (65, 5280, 4112),
+                                      (113, 5280, 4096), (128, 5280, 4112)])
 def test_streaming_form_at_ring_and_tile_edges(rows: int, k: int, n: int) -> None:
-    """K of 1, 3, 8, 9, 16 and 17 contraction steps (part of a chunk, part of a weight ring turn,
-    whole turns, one step more), 1 and 7 column tiles (a workgroup's last waves have none), rows
-    one past a tile, from a strided x and into a strided y: plain and gated."""
+    """The streaming form at 64 contraction steps (whole turns of its weight ring) and 165 (part of a
+    turn and of a chunk), column tiles that do not fill the last workgroup, rows one past a tile,
+    and two shapes beside them on the row kernel, from a strided x and into a strided y: plain and
+    gated."""
 
     from continuous_depth_batching_amd import ops
 
