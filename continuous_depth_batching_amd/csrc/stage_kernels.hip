@@ -480,18 +480,36 @@ __global__ void gate_state_reset_kernel(double* cdf, double* survival, float* pe
 // 64-bit divisions and its own read of the source. 48 tokens at 48 layers of 16
 // heads x 128 and 4 slots, 52 MB: 13.5 -> 11.6 us; 200 tokens 81 -> 51 us; 200 at 4
 // layers of 55 heads x 96 and 8 slots 37 -> 23 us; one token 3.3 -> 3.1 us.)
+// kPacked: rows under 4 KiB, `packed` (token, layer) pairs in a workgroup, whole rows side by
+// side (see cdb_exit_kv_copy).
 // ---------------------------------------------------------------------------
+template <bool kPacked>
 __global__ void __launch_bounds__(kThreads) exit_kv_copy_kernel(uint8_t* k_pool, uint8_t* v_pool,
                                                                int64_t layer_stride_bytes, int64_t row_bytes,
                                                                const int64_t* rows, const int32_t* exit_slot,
                                                                int64_t n, int32_t layer_base, int32_t core_layers,
-                                                               int32_t num_slots, int64_t pool_rows, int32_t per_group) {
+                                                               int32_t num_slots, int64_t pool_rows, int32_t per_group,
+                                                               int32_t packed) {
   const int64_t slot_bytes = core_layers * layer_stride_bytes;
-  const int64_t u = (int64_t)blockIdx.z * kThreads + threadIdx.x;
+  int64_t u = (int64_t)blockIdx.z * kThreads + threadIdx.x;
   const int first = 1 + blockIdx.y * per_group;
-  for (int64_t pair = blockIdx.x; pair < n * core_layers; pair += gridDim.x) {
-    const int64_t i = pair / core_layers;
-    const int l = (int)(pair - i * core_layers);
+  int local = 0;  // this thread's pair among the workgroup's
+  if constexpr (kPacked) {
+    const int units = (int)(row_bytes / 16);
+    local = threadIdx.x / units;
+    u = threadIdx.x - local * units;
+    if (local >= packed) return;
+  }
+  const int64_t step = kPacked ? packed : 1;
+  for (int64_t pair = blockIdx.x * step; pair < n * core_layers; pair += gridDim.x * step) {
+    int64_t i = pair / core_layers;  // uniform; a packed pair steps on from it in 32 bits
+    int l = (int)(pair - i * core_layers) + local;
+    if constexpr (kPacked) {
+      const int tokens = l / core_layers;
+      i += tokens;
+      l -= tokens * core_layers;
+      if (i >= n) continue;
+    }
     const int src_slot = exit_slot[i];
     const int64_t row = rows[i];
     const int end = min(first + per_group, num_slots - src_slot);
@@ -952,16 +970,29 @@ int cdb_exit_kv_copy(void* k_pool, void* v_pool, int64_t layer_stride, int64_t p
   // layers, 32 slots, 16 heads x 128: 5.6 us with all targets in one, 3.9 spread, 1 target per
   // workgroup up to 1024).
   constexpr int64_t kCopyBlocks = 1024;
-  const int64_t chunks = (row_bytes / 16 + kThreads - 1) / kThreads;
+  const int64_t units = row_bytes / 16;
+  const int64_t chunks = (units + kThreads - 1) / kThreads;
   const int64_t targets = num_slots - 1;
-  const int64_t spare = (n * core_layers * chunks * targets + kCopyBlocks - 1) / kCopyBlocks;
+  // A row under 4 KiB leaves threads idle, whose cost shows where a workgroup has little to store: its
+  // row and targets together under kThreads units. Packing whole rows side by side costs two 32-bit
+  // divisions a thread, some 0.15 us, so it starts at 32 pairs, or 256 (pair, target) copies, per unit
+  // of the row. (4 slots, 24 layers, one row a workgroup -> packed: 1 head x 64, 48 tokens 3.1 -> 2.8
+  // us, 4000 tokens 51 -> 11; 2 heads x 128, 200 tokens 5.7 -> 4.7, 4000 tokens 63 -> 39; one layer of
+  // 2 slots, 8 heads x 64, 4000 tokens 4.7 -> 3.8. Beyond the line: 8 heads x 64, 48 tokens and 24
+  // layers 3.4 -> 3.65; 32 slots and 4 layers of 4 heads x 96, 1000 tokens 17.5 -> 18.3.)
+  const int64_t pairs = n * core_layers;
+  const bool pack = units * num_slots <= kThreads && (pairs > 32 * units || pairs * targets > 256 * units);
+  const int64_t packed = pack ? kThreads / units : 1;
+  const int64_t blocks = (pairs + packed - 1) / packed;
+  const int64_t spare = (blocks * chunks * targets + kCopyBlocks - 1) / kCopyBlocks;
   const int64_t groups = spare >= targets ? 1 : (targets + spare - 1) / spare;
   const int64_t per_group = (targets + groups - 1) / groups;
   if (groups > 65535 || chunks > 65535) return CDB_ERR_SHAPE;
-  hipLaunchKernelGGL(exit_kv_copy_kernel, dim3(grid_for(n * core_layers, 1), (unsigned)groups, (unsigned)chunks),
-                     dim3(kThreads), 0, stream,
+  hipLaunchKernelGGL(pack ? exit_kv_copy_kernel<true> : exit_kv_copy_kernel<false>,
+                     dim3(grid_for(blocks, 1), (unsigned)groups, (unsigned)chunks), dim3(kThreads), 0, stream,
                      static_cast<uint8_t*>(k_pool), static_cast<uint8_t*>(v_pool), layer_stride * elem, row_bytes,
-                     rows, exit_slot, n, layer_base, core_layers, num_slots, pool_rows, (int32_t)per_group);
+                     rows, exit_slot, n, layer_base, core_layers, num_slots, pool_rows, (int32_t)per_group,
+                     (int32_t)packed);
   return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
 }
 
