@@ -579,7 +579,10 @@ constexpr int pow2_alignment(int bytes) { return bytes % 16 == 0 ? 16 : bytes % 
 template <typename T, int D, int C>
 CDB_DEVICE void rotate_chunk(const RopeWriteParams& P, const T* base, const T* bias, int pos, int chunk, float* out) {
   constexpr int kLanes = D / C, kHalfLanes = kLanes / 2;
-  const int partner_chunk = chunk < kHalfLanes ? chunk + kHalfLanes : chunk - kHalfLanes;
+  constexpr bool kPow2 = (kLanes & (kLanes - 1)) == 0;
+  const int partner_chunk = kPow2                ? chunk ^ kHalfLanes
+                            : chunk < kHalfLanes ? chunk + kHalfLanes
+                                                 : chunk - kHalfLanes;
   float own[C], partner[C];
   Vec<T, C> v;
   v.load(base + chunk * C);
@@ -615,7 +618,7 @@ CDB_DEVICE void rotate_chunk(const RopeWriteParams& P, const T* base, const T* b
   if (split_half) {
     // Elements d and d + D/2 share angle d mod D/2: the chunk's angles start at (chunk mod kHalfLanes) * C.
     float cs[C], sn[C];
-    const int f0 = (chunk < kHalfLanes ? chunk : chunk - kHalfLanes) * C;
+    const int f0 = (kPow2 ? chunk & (kHalfLanes - 1) : chunk < kHalfLanes ? chunk : chunk - kHalfLanes) * C;
     load_floats<C, pow2_alignment(C * 4)>(cr + f0, cs);
     load_floats<C, pow2_alignment(C * 4)>(sr + f0, sn);
     const bool low = chunk < kHalfLanes;
@@ -639,16 +642,15 @@ CDB_DEVICE void rotate_chunk(const RopeWriteParams& P, const T* base, const T* b
   }
 }
 
-// D / C lanes per head, C elements each: sixteenths of a head, or 16-byte units (see
-// launch_rope_write). What bounds a long prompt is the traffic, half reads and half writes.
-template <typename T, int D, int C>
+// 16 lanes per head (see launch_rope_write). What bounds a long prompt is the traffic, half reads
+// and half writes.
+template <typename T, int D>
 __global__ void __launch_bounds__(kThreads) rope_kv_write_kernel(RopeWriteParams P) {
-  constexpr int kLanes = D / C, kGroups = kThreads / kLanes;
-  const int local = threadIdx.x / kLanes;
-  const int64_t group = blockIdx.x * (int64_t)kGroups + local;
-  const int chunk = threadIdx.x - local * kLanes;
+  constexpr int C = D / 16, kGroups = kThreads / 16;
+  const int64_t group = blockIdx.x * (int64_t)kGroups + threadIdx.x / 16;
+  const int chunk = threadIdx.x & 15;
   const int64_t per_token = P.num_heads + P.num_kv_heads;
-  if (local >= kGroups || group >= P.tokens * per_token) return;
+  if (group >= P.tokens * per_token) return;
   const int64_t t = group / per_token;
   const int hh = (int)(group - t * per_token);
   const int pos = P.positions[t];
@@ -679,13 +681,60 @@ __global__ void __launch_bounds__(kThreads) rope_kv_write_kernel(RopeWriteParams
   if (row < 0 || row >= P.pool_rows || !rope_ok) return;
   float o[C];
   rotate_chunk<T, D, C>(P, static_cast<const T*>(P.k) + t * P.kv_stride + (int64_t)kvh * D,
-                     P.k_bias ? static_cast<const T*>(P.k_bias) + (int64_t)kvh * D : nullptr, pos, chunk, o);
+                        P.k_bias ? static_cast<const T*>(P.k_bias) + (int64_t)kvh * D : nullptr, pos, chunk, o);
   const int64_t off = (int64_t)P.layer * P.layer_stride + (row * P.num_kv_heads + kvh) * D + chunk * C;
   Vec<T, C> kw;
 #pragma unroll
   for (int i = 0; i < C; ++i) kw.set(i, o[i]);
   kw.store(static_cast<T*>(P.k_pool) + off);
   vv.store(static_cast<T*>(P.v_pool) + off);
+}
+
+// The same in 16-byte units, D / C lanes per head. The lanes of a head end anywhere in a wave, so most
+// waves hold query and key heads and rotate both on one path: as two branches they ran one after the
+// other, loads and all (55 heads x 96 in bf16, 4000 tokens 62 -> 58 us, 64 tokens 4.5 -> 4.0; 16 heads
+// x 128 in float, 1000 tokens 15.0 -> 13.8). Where a wave holds one kind the branches cost less, so
+// sixteenths keep them (12 + 4 heads x 64, 64 tokens 2.5 us against 2.7).
+template <typename T, int D>
+__global__ void __launch_bounds__(kThreads) rope_kv_write_units_kernel(RopeWriteParams P) {
+  constexpr int C = 16 / sizeof(T), kLanes = D / C, kGroups = kThreads / kLanes;
+  const int local = threadIdx.x / kLanes;
+  const int64_t group = blockIdx.x * (int64_t)kGroups + local;
+  const int chunk = threadIdx.x - local * kLanes;
+  const int64_t per_token = P.num_heads + P.num_kv_heads;
+  if (local >= kGroups || group >= P.tokens * per_token) return;
+  const int64_t t = group / per_token;
+  const int hh = (int)(group - t * per_token);
+  const int pos = P.positions[t];
+  const bool rope_ok = P.rope_style == 0 || (pos >= 0 && pos < P.max_positions);
+  const T* src = static_cast<const T*>(P.q) + t * P.q_stride + (int64_t)hh * D;
+  const T* bias = P.q_bias ? static_cast<const T*>(P.q_bias) + (int64_t)hh * D : nullptr;
+  T* dst = static_cast<T*>(P.q_out) + (t * P.num_heads + hh) * D + chunk * C;
+  T* v_dst = nullptr;
+  Vec<T, C> value;
+  if (hh >= P.num_heads) {
+    const int kvh = hh - P.num_heads;
+    value.load(static_cast<const T*>(P.v) + t * P.kv_stride + (int64_t)kvh * D + chunk * C);
+    const int64_t row = P.rows[t];
+    if (row < 0 || row >= P.pool_rows || !rope_ok) return;
+    const int64_t off = (int64_t)P.layer * P.layer_stride + (row * P.num_kv_heads + kvh) * D + chunk * C;
+    src = static_cast<const T*>(P.k) + t * P.kv_stride + (int64_t)kvh * D;
+    bias = P.k_bias ? static_cast<const T*>(P.k_bias) + (int64_t)kvh * D : nullptr;
+    dst = static_cast<T*>(P.k_pool) + off;
+    v_dst = static_cast<T*>(P.v_pool) + off;
+  }
+  float o[C];
+  if (rope_ok) {
+    rotate_chunk<T, D, C>(P, src, bias, pos, chunk, o);
+  } else {
+#pragma unroll
+    for (int i = 0; i < C; ++i) o[i] = __builtin_nanf("");
+  }
+  Vec<T, C> rotated;
+#pragma unroll
+  for (int i = 0; i < C; ++i) rotated.set(i, o[i]);
+  rotated.store(dst);
+  if (v_dst) value.store(v_dst);
 }
 
 }  // namespace cdb
@@ -714,22 +763,24 @@ int launch_norm(const NormParams& P, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
 }
 
-template <typename T, int D, int C>
-int launch_rope_write_chunks(const RopeWriteParams& P, hipStream_t s) {
-  constexpr int kGroups = kThreads / (D / C);
-  const int64_t blocks = (P.tokens * (P.num_heads + P.num_kv_heads) + kGroups - 1) / kGroups;
+int launch_rope_write(void (*kernel)(RopeWriteParams), int64_t groups, const RopeWriteParams& P, hipStream_t s) {
+  const int64_t blocks = (P.tokens * (P.num_heads + P.num_kv_heads) + groups - 1) / groups;
   if (blocks > 0x7fffffff) return CDB_ERR_SHAPE;
-  hipLaunchKernelGGL((rope_kv_write_kernel<T, D, C>), dim3((unsigned)blocks), dim3(kThreads), 0, s, P);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kThreads), 0, s, P);
   return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
 }
 
 // Sixteenths of a head are 8 or 16 bytes for bf16 heads of 64 and 128 and float heads of 64: one
 // access per lane and row part. The other heads (12 bytes, three 4-byte accesses; 24 and 32
 // bytes, several with gaps between the lanes) take 16-byte units where everything is aligned to
-// them: 55 heads x 96 in bf16, 4000 tokens, 70 -> 62 us and 512 or fewer the same (10 us); 16 heads
-// x 128 in float, 4000 tokens, 54 -> 47 us, 100 tokens 3.6 -> 3.3. (8-byte sixteenths in 16-byte
-// units were slower: 12 + 4 heads x 64, 2000 tokens, 5.0 -> 7.2 us.) The halves of a head
-// may then lie in different waves, so what is read must not be what is written.
+// them: 55 heads x 96 in bf16, 4000 tokens, 70 -> 58 us, 64 tokens 4.3 -> 4.0; 16 heads
+// x 128 in float, 4000 tokens, 54 -> 45 us, 100 tokens 3.6 -> 3.3. (8-byte sixteenths in 16-byte
+// units were slower: 12 + 4 heads x 64, 2000 tokens, 5.0 -> 7.2 us.) Not so in bf16 while the launch is
+// latency and each wave of sixteenths (four heads) is of one kind: 16 + 4 heads, 64 tokens 2.65 us
+// against 2.95 in units, 1000 tokens (20,000 heads) 4.7 against 4.9, 2000 tokens 9.1 against 7.6; 16 +
+// 16 heads, 64 tokens 2.9 against 3.2, 1000 tokens (32,000) 8.3 against 7.3. The halves of a head
+// may lie in different waves in units, so what is read must not be what is written.
+constexpr int64_t kRopeFewHeads = 24576;
 template <typename T, int D>
 int launch_rope_write(const RopeWriteParams& P, hipStream_t s) {
   constexpr int64_t kElem = sizeof(T);
@@ -747,9 +798,12 @@ int launch_rope_write(const RopeWriteParams& P, hipStream_t s) {
     const bool apart = !overlap(P.q, P.q_stride, P.num_heads, P.q_out, 0, P.tokens * P.num_heads * D * kElem) &&
                        !overlap(P.k, P.kv_stride, P.num_kv_heads, P.k_pool, pool_at, pool_bytes) &&
                        !overlap(P.v, P.kv_stride, P.num_kv_heads, P.v_pool, pool_at, pool_bytes);
-    if (apart && ((at | strides) & 15) == 0) return launch_rope_write_chunks<T, D, 16 / kElem>(P, s);
+    const bool few = sizeof(T) == 2 && P.num_heads % 4 == 0 && P.num_kv_heads % 4 == 0 &&
+                     P.tokens * (P.num_heads + P.num_kv_heads) < kRopeFewHeads;
+    if (!few && apart && ((at | strides) & 15) == 0)
+      return launch_rope_write(rope_kv_write_units_kernel<T, D>, kThreads / (D * kElem / 16), P, s);
   }
-  return launch_rope_write_chunks<T, D, D / 16>(P, s);
+  return launch_rope_write(rope_kv_write_kernel<T, D>, kThreads / 16, P, s);
 }
 
 }  // namespace

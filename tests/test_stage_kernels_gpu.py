@@ -401,6 +401,36 @@ def test_rope_kv_write_in_16_byte_units(dtype: str, head_dim: int, style: int) -
     assert bool((outs[0][1][1, 0, 8] != 0).any()) and bool((outs[0][0][3] == 1e30).all()) == (style != 0)
 
 
+@pytest.mark.parametrize("style", [0, 1, 2])
+def test_rope_kv_write_gives_a_token_the_same_bits_in_short_and_long_prompts(style: int) -> None:
+    """96-wide bf16 heads, four of a kind to a wave: a launch of 24,576 heads or more takes 16-byte
+    units, a shorter one sixteenths. Tokens of the long launch agree with launches of the first, the
+    last and one short of that line."""
+
+    from continuous_depth_batching_amd import ops
+
+    torch.manual_seed(style)
+    heads, kv_heads, dim, bs, tokens = 16, 4, 96, 16, 1250
+    mk = lambda n, *shape: torch.randn(n, *shape, device="cuda").bfloat16()
+    q, k, v = mk(tokens, heads, dim), mk(tokens, kv_heads, dim), mk(tokens, kv_heads, dim)
+    qb, kb = mk(heads, dim), mk(kv_heads, dim)
+    cos, sin = torch.randn(tokens, dim // 2, device="cuda"), torch.randn(tokens, dim // 2, device="cuda")
+    rows = torch.randperm(tokens, device="cuda")
+    pos = torch.randperm(tokens, device="cuda").int()
+
+    def write(at: slice) -> tuple[torch.Tensor, torch.Tensor]:
+        pool = torch.zeros(1, 2, 1264, kv_heads, dim, dtype=torch.bfloat16, device="cuda")
+        out = torch.empty_like(q[at])
+        ops.rope_kv_write_raw(q[at], k[at], v[at], out, ops.KVPoolView(pool, bs), 0, rows[at].contiguous(),
+                              pos[at].contiguous(), cos, sin, style, qb, kb)
+        return out, pool[0][:, rows[at]]
+
+    whole_q, whole_kv = write(slice(0, tokens))
+    for at in (slice(0, 1), slice(tokens - 33, tokens), slice(0, 24576 // 20), slice(0, 24576 // 20 + 1)):
+        out, kv = write(at)
+        assert torch.equal(out, whole_q[at]) and torch.equal(kv, whole_kv[:, at])
+
+
 @pytest.mark.parametrize("head_dim", [64, 96, 128])
 @pytest.mark.parametrize("split", [False, True])
 def test_prefill_attention_does_not_depend_on_the_page_size(head_dim: int, split: bool) -> None:
