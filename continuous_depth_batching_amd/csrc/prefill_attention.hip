@@ -499,9 +499,11 @@ __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillPara
   // SIMD's oldest wave, so its workgroups finish one after the other and the last run alone.
   // A part's priority falls with the blocks it has left, which keeps the workgroups of a CU
   // abreast (4 x 128 queries after 16,000 keys: 123 -> 118 us). Whole tiles, of all lengths,
-  // are refilled from the rest of the launch and do not gain (49.7 -> 50.7 us).
+  // are refilled from the rest of the launch and do not gain (49.7 -> 50.7 us); they pay one compare
+  // a block. Heads of 96 go without: 55 heads, 128 queries after 16,000 keys 126 us with it and 120
+  // without, though 16 heads, 4 x 128 queries after 8000 keys, 66 and 68.
+  const bool steps_priority = D != 96 && slot >= 0;
   auto set_priority = [&](int left) {
-    if (slot < 0) return;
     if (left >= 24) __builtin_amdgcn_s_setprio(3);
     else if (left >= 12) __builtin_amdgcn_s_setprio(2);
     else if (left >= 4) __builtin_amdgcn_s_setprio(1);
@@ -518,10 +520,17 @@ __global__ void __launch_bounds__(256) prefill_attention_bf16_kernel(PrefillPara
   } else {
     __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
-  set_priority(num_blocks - block0);
+  int priority_step = num_blocks;  // the block at which the priority changes next
+  if (steps_priority) {
+    const int left = num_blocks - block0;
+    set_priority(left);
+    priority_step -= left > 23 ? 23 : left > 11 ? 11 : 3;
+  }
   for (int b = block0; b < num_blocks; ++b) {
-    const int left = num_blocks - b;
-    if (left == 23 || left == 11 || left == 3) set_priority(left);
+    if (b == priority_step) {
+      set_priority(num_blocks - b);
+      priority_step = num_blocks - (num_blocks - b == 23 ? 11 : 3);
+    }
     // Block b has landed once at most block b + 1's loads are outstanding.
     if (b > block0) {
       if (b + 1 < num_blocks) {
