@@ -248,7 +248,6 @@ __global__ void __launch_bounds__(MAXT) linear_kernel(LinearParams p) {
 // against 11.6 / 12.1. Above those rows it is the faster one (see dispatch_parts).
 // ---------------------------------------------------------------------------
 constexpr int kPartsStages = 4;
-constexpr int kPartsSteps = 4;  // steps per chunk
 
 // Slot of x unit (row r of a 16-row tile, step t of the chunk, k group g) within
 // its 64-unit block: the MFMA lane that reads it is r + 16 g, with r swizzled by
@@ -258,11 +257,12 @@ constexpr int kPartsSteps = 4;  // steps per chunk
 // stay conflict-free.
 CDB_DEVICE int x_slot(int r, int t, int g) { return (r ^ (4 * (t & 3) + g)) + 16 * g; }
 
+// SC: contraction steps per chunk.
 // NTAIL: N is a multiple of 16 but not of 64, so the last column range is narrower;
 // without it N must be a multiple of 64.
-template <int MT, int KSTEPS, int KSPLIT, bool NTAIL>
+template <int MT, int SC, int KSTEPS, int KSPLIT, bool NTAIL>
 __global__ void __launch_bounds__(256) linear_parts_kernel(LinearParams p) {
-  constexpr int SC = kPartsSteps, STAGES = kPartsStages;
+  constexpr int STAGES = kPartsStages;
   constexpr int ROWS = 16 * MT;
   constexpr int KC = 32 * SC;
   constexpr int UPT = ROWS * KC / 8 / 256;  // x units per thread and chunk
@@ -366,12 +366,12 @@ __global__ void __launch_bounds__(256) linear_parts_kernel(LinearParams p) {
   }
 }
 
-template <int MT, int KSTEPS, int KSPLIT, bool NTAIL = false>
+template <int MT, int SC, int KSTEPS, int KSPLIT, bool NTAIL = false>
 int launch_linear_parts(LinearParams prm, hipStream_t stream) {
   if ((NTAIL ? prm.N % 16 : prm.N % 64) || prm.K != 32 * KSTEPS * KSPLIT) return CDB_ERR_SHAPE;
   const int n_tiles = NTAIL ? (prm.N / 16 + 3) / 4 : prm.N / 64;  // as the kernel counts
   const int m_tiles = (prm.M + 16 * MT - 1) / (16 * MT);
-  hipLaunchKernelGGL((linear_parts_kernel<MT, KSTEPS, KSPLIT, NTAIL>),
+  hipLaunchKernelGGL((linear_parts_kernel<MT, SC, KSTEPS, KSPLIT, NTAIL>),
                      dim3((n_tiles * KSPLIT + 7) / 8 * 8 * m_tiles), dim3(256), 0, stream, prm);
   return hipGetLastError() == hipSuccess ? CDB_OK : CDB_ERR_HIP;
 }
@@ -406,6 +406,7 @@ int launch_linear_parts(LinearParams prm, hipStream_t stream) {
 constexpr int kStreamSteps = 4;        // SC: contraction steps per x chunk (256 bytes of a row)
 constexpr int kStreamRing = 8;         // RW: weight steps in flight per consumer wave
 constexpr int kStreamMaxConsumers = 6;
+constexpr int kStreamCus = 256;        // CUs the tile and form choices spread workgroups over
 // S: x stages in LDS. A stage is MT * SC KiB; eight row tiles fit three (and keep the
 // producer's loads in flight under the 63 a wave can count).
 template <int MT> constexpr int kStreamStages = MT < 8 ? 4 : 3;
@@ -795,7 +796,7 @@ StreamTile choose_stream_tile(const LinearParams& prm, StreamMode mode, int spli
         const int cols = c * ntw;
         if (ntw == 2 && cols <= kStreamMaxConsumers) continue;  // one tile per wave covers it
         const int64_t groups = (int64_t)((col_tiles + cols - 1) / cols) * splits * ((row_tiles + mt - 1) / mt);
-        const int64_t cost = (groups + 255) / 256 * (mt + cols * (mode == StreamMode::kGated ? 2 : 1));
+        const int64_t cost = (groups + kStreamCus - 1) / kStreamCus * (mt + cols * (mode == StreamMode::kGated ? 2 : 1));
         if (cost <= best_cost) {  // a tie goes to the taller tile: fewer row ranges re-read W from L2
           best_cost = cost;
           best = StreamTile{mt, ntw, c};
@@ -851,18 +852,37 @@ int parts_splits(int64_t rows, int32_t out_features, int32_t in_features) {
   return 0;
 }
 
-// The few-row form where it measured faster (figures at its kernel); from the next width up the
-// streaming form is: 2048 -> 2048 at 90 rows 5.8 -> 5.5 us, 5632 -> 2048 at 90 / 200 rows
-// 9.1 -> 8.9 / 13.5 -> 12.0, 5280 -> 5280 at 100 rows 23.1 -> 17.1, 17920 -> 5280 at
-// 32 / 100 rows 38.6 -> 34.1 / 78 -> 42.
+// Whether the few-row form with row ranges of 16 * mt rows gives nearly every CU one workgroup and
+// none a second: from `least` workgroups to kStreamCus.
+bool fills_cus_once(const LinearParams& prm, int splits, int mt, int least) {
+  const int groups = (prm.N / 16 + 3) / 4 * splits * ((prm.M + 16 * mt - 1) / (16 * mt));
+  return groups >= least && groups <= kStreamCus;
+}
+
+// The few-row form where it measured faster than the streaming form's chosen tile: up to the row counts
+// of the first lines whatever the width (figures at its kernel), and above where its workgroups fill
+// the CUs once. us, few-row / streaming:
+//   5280 -> 5280, 249 workgroups: 17 rows 11.5 / 12.3, 32 11.9 / 12.7, 48 13.0 / 13.7, 64 14.3 / 14.6
+//   5280 -> 4096 (192) 24 rows 10.5 / 11.0; -> 3584 (168) 10.3 / 10.2; -> 2048 (96) 9.7 / 8.3
+//   2048 -> 2048, 97 and 128 rows (256): 5.5 / 5.5, 5.7 / 5.8; 65 and 96 rows (192) 5.4 / 5.1, 5.65 / 5.35
+//   5632 -> 2048, 65 rows (256): 8.7 / 8.6, 80 8.8 / 9.0, 104 9.0 / 9.2, 128 9.5 / 9.8;
+//   5632 -> 1536 (192) 96 rows 8.5 / 8.1
+// With a second round of workgroups the streaming form is faster: 5280 -> 5280 at 100 rows 23.1 / 17.1,
+// 5632 -> 2048 at 200 rows 13.5 / 12.0, 17920 -> 5280 at 32 / 100 rows 38.6 / 34.1 and 78 / 42.
 int dispatch_parts(const LinearParams& prm, int splits, hipStream_t stream) {
-  if (prm.K == 2048 && prm.M <= 32) return launch_linear_parts<1, 16, 4>(prm, stream);
-  if (prm.K == 2048 && prm.M <= 64) return launch_linear_parts<2, 16, 4>(prm, stream);
-  if (prm.K == 5632 && prm.M <= 16) return launch_linear_parts<1, 22, 8>(prm, stream);
-  if (prm.K == 5632 && prm.M <= 32) return launch_linear_parts<1, 44, 4>(prm, stream);
-  if (prm.K == 5632 && prm.M <= 64) return launch_linear_parts<2, 44, 4>(prm, stream);
-  if (prm.K == 5280 && prm.M <= 16) return launch_linear_parts<1, 55, 3, true>(prm, stream);
-  if (prm.K == 17920 && prm.M <= 16) return launch_linear_parts<1, 70, 8, true>(prm, stream);
+  if (prm.K == 2048 && prm.M <= 32) return launch_linear_parts<1, 4, 16, 4>(prm, stream);
+  if (prm.K == 2048 && prm.M <= 64) return launch_linear_parts<2, 4, 16, 4>(prm, stream);
+  if (prm.K == 5632 && prm.M <= 16) return launch_linear_parts<1, 4, 22, 8>(prm, stream);
+  if (prm.K == 5632 && prm.M <= 32) return launch_linear_parts<1, 4, 44, 4>(prm, stream);
+  if (prm.K == 5632 && prm.M <= 64) return launch_linear_parts<2, 4, 44, 4>(prm, stream);
+  if (prm.K == 5280 && prm.M <= 16) return launch_linear_parts<1, 4, 55, 3, true>(prm, stream);
+  if (prm.K == 17920 && prm.M <= 16) return launch_linear_parts<1, 4, 70, 8, true>(prm, stream);
+  if (prm.K == 5280 && prm.M <= 64 && fills_cus_once(prm, splits, 4, 192))
+    return launch_linear_parts<4, 2, 55, 3, true>(prm, stream);
+  if (prm.K == 2048 && prm.M <= 128 && fills_cus_once(prm, splits, 2, 196))
+    return launch_linear_parts<2, 4, 32, 2>(prm, stream);
+  if (prm.K == 5632 && prm.M <= 128 && fills_cus_once(prm, splits, 4, 196))
+    return launch_linear_parts<4, 2, 44, 4>(prm, stream);
   return dispatch_stream(prm, StreamMode::kParts, splits, stream);
 }
 

@@ -300,6 +300,34 @@ def test_streamed_partials_at_row_range_edges(rows: int, k: int, n: int) -> None
         assert ((parts[s] - xs @ ws.t()).abs() <= (xs.abs() @ ws.abs().t()) * 2.0 ** -16).all()
 
 
+@pytest.mark.parametrize("k,n,rows", [(5280, 5280, (17, 33, 64, 65)), (5280, 4096, (17, 64)), (5280, 4032, (64,)),
+                                      (2048, 2048, (65, 96, 97, 128)), (2048, 2560, (65, 96, 97)),
+                                      (5632, 2048, (65, 81, 128, 129)), (5632, 1600, (65, 128))])
+def test_split_k_forms_agree_where_the_shape_changes_them(k: int, n: int, rows: tuple[int, ...]) -> None:
+    """Row counts and widths on both sides of the lines between the few-row and the streaming form.
+    Both add a K range's steps in order in one accumulator, so a row's partials have the bits of the
+    largest batch with the same ranges (streaming: 256 rows, or 128 for a 2048-wide input)."""
+
+    from continuous_depth_batching_amd import ops
+
+    most = 128 if k == 2048 else 256
+    x, w = _inputs(most, k, n, seed=k + n)
+    packed = ops.pack_linear_weight(w)
+
+    def partials(r: int) -> torch.Tensor:
+        parts = torch.full((ops.linear_parts_splits(r, n, k), r, n), float("nan"), device="cuda")
+        ops.linear_parts_raw(x[:r], packed, parts)
+        return parts
+
+    whole = partials(most)
+    for r in rows:
+        assert ops.linear_parts_splits(r, n, k) == whole.shape[0]
+        assert torch.equal(partials(r), whole[:, :r]), r
+    width = k // whole.shape[0]
+    xs, ws = x[:, :width].float(), w[:, :width].float()
+    assert ((whole[0] - xs @ ws.t()).abs() <= (xs.abs() @ ws.abs().t()) * 2.0 ** -16).all()
+
+
 @pytest.mark.parametrize("rows,k,n", [(1, 2048, 2048), (16, 5632, 2048), (33, 2048, 2048), (96, 5632, 2048),
                                       (128, 2048, 2048), (256, 5632, 2048), (7, 5280, 5280), (128, 17920, 5280)])
 def test_norm_from_partials_is_the_two_step_result(rows: int, k: int, n: int) -> None:
