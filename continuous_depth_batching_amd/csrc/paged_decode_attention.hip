@@ -27,8 +27,8 @@
 //       shape): each wave keeps one or two K/V steps in flight besides the one it
 //       computes, and the wave that stores a row's last chunk merges the row
 //       (arrival counters, agent-coherent partials).
-//     - paged_decode_fast_kernel (the same shape, more than kPersistentRows rows of
-//       64-wide heads): while a wave streams one item it already holds the next
+//     - paged_decode_fast_kernel (the same shape, many rows of 64-wide heads, see
+//       kPersistentRows): while a wave streams one item it already holds the next
 //       item's descriptor and loads its query and new token, and the next item's
 //       first K/V step is issued into the buffer the current item's last step
 //       frees; the launch's tail goes to whichever wave asks first, from its XCD's
@@ -1152,7 +1152,16 @@ template <int D> constexpr int kDeepRowsOf = D == 128 ? 256 : 120;
 // at 256 rows, 309 against 327 at 512, 368 against 389 at 1000). At 128 wide it took 461 us
 // against 431 at 512 rows and 433 against 406 at 1024; at 55 heads x 96 606 against 580 at 128
 // rows; in float at 16 x 128, where it spills, 6.5 ms against 3.1 at 300 rows of 1500-2000 tokens.
+// Between kDeepRowsOf and that many rows the contexts decide, of which the host knows only the most
+// the table holds. bf16, persistent / deep: 12 heads, 128 rows of 64-900 tokens 82 / 70 us, 900-1100
+// 171 / 162, 1500-2000 259 / 268, 3000-4000 501 / 551; 256 rows 131 / 115, 296 / 298, 498 / 521,
+// 1002 / 1086, 1400-1500 439 / 465; 8 heads on 4, 256 rows 93 / 73, 185 / 185, 303 / 318, 603 / 651. In
+// float the line lies twice as far for 12 heads (256 rows of 1400-1500 824 / 805, 3000-4000 1829 /
+// 1894) and nowhere for shared ones (8 on 4, 3000-4000: 1068 / 1008). So the persistent form takes
+// tables of more than kPersistentPages pages, in float twice that and with a K/V head per query head;
+// short contexts under a wide table then run the slower form.
 constexpr int kPersistentRows = 256;
+constexpr int kPersistentPages = 72;
 
 template <typename T, int D, bool kCoherent = false>
 CDB_DEVICE void merge_chunks(const float* part, int64_t stride, int nsplit, int lane, T* out_row);
@@ -1518,10 +1527,15 @@ int launch_decode(const DecodeParams& P, int stages, int num_cus, hipStream_t st
   DecodeKernel kernel = paged_decode_kernel<T, D, R>;
   bool merged = false;
   if (fast_form(P)) {
-    merged = D != 64 || P.num_rows <= kPersistentRows;
     kernel = P.num_rows <= kDeepRowsOf<D> ? paged_decode_deep_kernel<T, D, R, 3> : paged_decode_deep_kernel<T, D, R, 2>;
+    merged = true;
     if constexpr (D == 64) {
-      if (!merged) kernel = paged_decode_fast_kernel<T, D, R>;
+      const bool shared_float = sizeof(T) == 4 && P.num_kv_heads < P.num_heads;
+      if (P.num_rows > kPersistentRows ||
+          (P.num_rows > kDeepRowsOf<D> && P.table_width > kPersistentPages * (int)sizeof(T) / 2 && !shared_float)) {
+        kernel = paged_decode_fast_kernel<T, D, R>;
+        merged = false;
+      }
     }
   }
   const int rc = launch_persistent(kernel, P, num_cus, stream);

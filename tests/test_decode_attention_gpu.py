@@ -187,6 +187,13 @@ def _device_case(case):
     return tensors, ws
 
 
+def _holds_every_chunk(case) -> bool:
+    """Whether _device_case's workspace holds a chunk per 8 pages of the table, as the deep and the
+    persistent form need (the general form runs otherwise)."""
+
+    return -(-case.block_table.shape[1] // 8) <= -(-(int(case.seqlens.max()) + 1) // 128)
+
+
 def _attend(case, d, ws, rows, cache_layer0=0, stages=None):
     """Decode attention over the batch rows `rows` (indices into the case) through table_row."""
     from continuous_depth_batching_amd import ops
@@ -256,6 +263,54 @@ def test_forms_agree_where_the_row_count_changes_them(dtype: str, heads: int, he
     few = _attend(case, d, ws, list(range(20)))
     torch.cuda.synchronize()
     assert torch.equal(less, full[1:]) and torch.equal(few, full[:20])
+
+
+@pytest.mark.parametrize("dtype,heads,kv_heads,rows", [("bf16", 2, 2, 121), ("bf16", 4, 2, 256), ("f32", 2, 2, 256),
+                                                       ("f32", 2, 1, 121)])
+def test_forms_agree_where_the_table_width_changes_them(dtype: str, heads: int, kv_heads: int, rows: int) -> None:
+    """64-wide heads between 121 and 256 rows: tables of more than 72 pages (144 in float) run the
+    persistent form, though not in float with shared heads, narrower ones the deep form, and few rows the deep form with
+    three buffers. The same bits in each, with contexts that fit the narrow table."""
+
+    case = make_case(seed=rows + heads, num_rows=rows, num_heads=heads, num_kv_heads=kv_heads, head_dim=64,
+                     max_context=480, rope_style=1, dtype=dtype, padding_rows=2, num_layers=2)
+    d, ws = _device_case(case)
+    assert _holds_every_chunk(case)
+    narrow = _attend(case, d, ws, list(range(rows)))
+    more = (73 if dtype == "bf16" else 145) - d["table"].shape[1]
+    d["table"] = torch.nn.functional.pad(d["table"], (0, more), value=-1)
+    wide_ws = torch.empty(5 * ws.numel(), device="cuda")  # a chunk per 8 pages of the wide table
+    wide = _attend(case, d, wide_ws, list(range(rows)))
+    few = _attend(case, d, wide_ws, list(range(20)))
+    torch.cuda.synchronize()
+    assert torch.equal(wide, narrow) and torch.equal(few, narrow[:20])
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("rope_style", [0, 1, 2])
+def test_persistent_form_over_several_rounds(dtype: str, rope_style: int) -> None:
+    """The persistent form with some five items a wave: rounds that prefetch the next item, the LDS
+    stash's both halves, and the tail queues. Against the oracle, with q/k bias beside the interleaved
+    rotation, and bit for bit against the deep form (the first 100 rows alone)."""
+
+    case = make_case(seed=41 + rope_style, num_rows=300, num_heads=32, num_kv_heads=2, head_dim=64, max_context=480,
+                     rope_style=rope_style or 1, dtype=dtype, padding_rows=3, num_layers=1, qk_bias=rope_style == 2)
+    case.rope_style = rope_style
+    d, ws = _device_case(case)
+    if not rope_style:
+        case.rope = d["cos"] = d["sin"] = None
+    chunks = int(np.sum(case.seqlens[case.seqlens >= 0] // 128 + 1))
+    assert _holds_every_chunk(case) and chunks * 32 > 4 * 4096  # resident waves: 3072 in float, 4096 in bf16
+    out = _attend(case, d, ws, list(range(300)))
+    pool = d["pool"].float().cpu().numpy()
+    first = _attend(case, d, ws, list(range(100)))
+    torch.cuda.synchronize()
+    assert torch.equal(first, out[:100])
+    want, want_pool = run_oracle(case)
+    err = np.abs(out.float().cpu().numpy() - want)
+    max_tol, mean_tol = TOL[dtype]
+    assert err.max() <= max_tol and err.mean() <= mean_tol, (err.max(), err.mean())
+    np.testing.assert_array_equal(pool, want_pool)
 
 
 FAST_FORM_SHAPES = {
