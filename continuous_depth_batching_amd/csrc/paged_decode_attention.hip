@@ -1145,7 +1145,11 @@ __global__ void __launch_bounds__(256, 3) paged_decode_fast_kernel(DecodeParams 
 // Up to kDeepRowsOf<D> rows a wave has a few items and latency counts: three buffers (16 rows of 12
 // heads x 64, two layers with the plan: 38.1 us against 40.4 with two; 256 rows of 16 x 128: 363
 // against 374, and 387 with four). Above, two leave room for more waves (512 rows of 16 x 128: 431
-// us against 448 with three; 1024: 406 against 420).
+// us against 448 with three; 1024: 406 against 420). Three buffers of a float head of 128 need more than
+// the 256 registers (16-29 spilled), so with a rotation's angles beside them it takes two throughout:
+// two layers of 16 x 128, 16 rows of 64-900 tokens 70 against 67 us, 256 rows 559 against 526, of 8-64
+// 119 against 100. (Without rotation three still read faster where heads share: 32 on 8 heads, 256 rows
+// of 1500-2000, 3925 against 4078.)
 template <int D> constexpr int kDeepRowsOf = D == 128 ? 256 : 120;
 // The persistent form stays where its prefetch across items still pays: many rows of 64-wide
 // heads, whose items are half as long (12 heads, two layers: 174 us against 171 with the deep form
@@ -1527,7 +1531,11 @@ int launch_decode(const DecodeParams& P, int stages, int num_cus, hipStream_t st
   DecodeKernel kernel = paged_decode_kernel<T, D, R>;
   bool merged = false;
   if (fast_form(P)) {
-    kernel = P.num_rows <= kDeepRowsOf<D> ? paged_decode_deep_kernel<T, D, R, 3> : paged_decode_deep_kernel<T, D, R, 2>;
+    constexpr bool kSpills = sizeof(T) == 4 && D == 128 && R != 0;  // with three buffers
+    kernel = paged_decode_deep_kernel<T, D, R, 2>;
+    if constexpr (!kSpills) {
+      if (P.num_rows <= kDeepRowsOf<D>) kernel = paged_decode_deep_kernel<T, D, R, 3>;
+    }
     merged = true;
     if constexpr (D == 64) {
       const bool shared_float = sizeof(T) == 4 && P.num_kv_heads < P.num_heads;
