@@ -67,8 +67,9 @@ def test_linear_matches_rounded_fp32_product(rows: int, k: int, n: int) -> None:
 
 @pytest.mark.parametrize("rows,k,n", [(r, 2048, n) for r in (33, 65, 96, 128, 129, 200, 256) for n in (6144, 4096)]
                          + [(r, 5280, 15840) for r in (65, 100, 128)])
-def test_wide_tile_path_matches_rounded_fp32_product(rows: int, k: int, n: int) -> None:
-    """Batches above 32 rows with 2048-wide inputs and 4096+ outputs take the wide-tile kernel."""
+def test_streaming_path_matches_rounded_fp32_product(rows: int, k: int, n: int) -> None:
+    """Batches above 32 rows with 2048-wide inputs and 4096+ outputs, and above 64 with 5280-wide
+    ones, take the streaming kernel."""
 
     from continuous_depth_batching_amd import ops
 
@@ -85,7 +86,7 @@ def test_gated_linear_follows_bf16_silu_chain(rows: int, k: int, f: int) -> None
     from continuous_depth_batching_amd import ops
 
     if rows > ops.LINEAR_MAX_ROWS and not ops.linear_prefers_kernel(rows, f, True, k):
-        pytest.skip("above 64 rows only the wide-tile shapes run on cdb_linear")
+        pytest.skip("above 64 rows only the streaming shapes run on cdb_linear")
 
     x, w = _inputs(rows, k, 2 * f, seed=rows + f)
     y = torch.empty((rows, f), dtype=torch.bfloat16, device="cuda")
@@ -114,7 +115,7 @@ def test_fused_silu_gives_torch_bits_for_every_normal_bf16_gate(rows: int) -> No
     weight and every up value exactly 1, and each output is the SiLU of that bf16 value
     alone. Across the batch every finite normal bf16 value (and +0) is a gate once; each
     output must equal torch's bf16 SiLU bit for bit (the row kernel at 16 rows, the
-    pipelined wide-tile forms at 100 and 256)."""
+    streaming kernel with four and eight row tiles at 100 and 256)."""
 
     from continuous_depth_batching_amd import ops
 
@@ -224,12 +225,12 @@ def test_split_k_partials_sum_to_the_fp32_product(rows: int, k: int, n: int) -> 
     _check_rounded(total.bfloat16(), x.float() @ w.float().t(), max_mismatch=0.01, extra=_sum_error(x, w))
 
 
-def test_wide_tile_forms_give_a_row_the_same_bits_in_any_batch() -> None:
-    """Every wide-tile form adds an output's K steps in order in one accumulator, so a
-    row's result does not depend on its batch: 48 rows (two-tile row ranges), 100 rows
-    (four-tile; the gated one reads x ahead of its MFMAs) and 256 rows (eight-tile gated
-    and down forms, both reading x ahead) agree bit for bit, for the gated projection and
-    for the split-K partials. A dropped, repeated or reordered K step in one form fails."""
+def test_a_row_has_the_same_bits_in_any_streamed_batch() -> None:
+    """The streaming kernel and the few-row split-K form add an output's K steps (of a range) in order
+    in one accumulator, so a row's result does not depend on its batch: the gated projection at 48
+    (three row tiles), 100 (four) and 256 rows (eight), and the split-K partials at 48 and 100 rows
+    (few-row form) and 256 (streamed) agree bit for bit. A dropped, repeated or reordered K step in
+    one of them fails."""
 
     from continuous_depth_batching_amd import ops
 
@@ -253,14 +254,68 @@ def test_wide_tile_forms_give_a_row_the_same_bits_in_any_batch() -> None:
     assert ((gated[256].float() - ref).abs() <= 2 * _bf16_ulp(ref) + 1e-3).float().mean().item() >= 0.99
 
 
+# (mode, in, out, rows): at these row counts the streaming kernel runs every tile it is given for the
+# Ouro-1.4B and Huginn-0125 projections. Row tiles, and column tiles per wave where there are two:
+STREAMED = [
+    ("plain", 2048, 6144, (40, 64, 100, 150, 177, 215, 256)),   # 3, 2, 4, 5, 6, 7, 4
+    ("plain", 5280, 15840, (70, 90, 105, 128)),                 # 5, 6, 7, 8
+    ("gated", 2048, 5632, (40, 100, 150, 177, 215, 256)),       # 3, 4, 5, 6, 7, 8
+    ("gated", 5280, 17920, (70, 90, 105, 128)),                 # 5, 6, 7, 8
+    ("parts", 2048, 2048, (90, 128)),                           # 3, few-row form
+    ("parts", 5632, 2048, (20, 150, 177, 215, 256)),            # few-row form, 5, 6, 7, 8
+    ("parts", 5280, 5280, (20, 70, 90, 105, 128, 150, 177, 215, 256)),   # few-row form, 5 to 8, 5 x 2 to 8 x 2
+    ("parts", 17920, 5280, (20, 40, 60, 64)),                   # eight ranges: 2 x 2, 3 x 2, 4 x 2
+    ("parts", 17920, 5280, (70, 90, 105, 128, 150, 177, 215, 256)),      # four: 5 to 8, 5 x 2 to 8 x 2
+]
+
+
+@pytest.mark.parametrize("mode,k,n,rows", STREAMED)
+def test_every_streaming_tile_has_the_bits_of_the_largest_batch(mode: str, k: int, n: int,
+                                                               rows: tuple[int, ...]) -> None:
+    """Each batch against the largest of its line, and that one against the fp32 product."""
+
+    from continuous_depth_batching_amd import ops
+
+    x, w = _inputs(rows[-1], k, (2 if mode == "gated" else 1) * n, seed=k + n + len(rows))
+    packed = ops.pack_linear_weight(w)
+
+    def project(r: int) -> torch.Tensor:
+        if mode == "parts":
+            out = torch.full((ops.linear_parts_splits(r, n, k), r, n), float("nan"), device="cuda")
+            ops.linear_parts_raw(x[:r], packed, out)
+            return out.transpose(0, 1)
+        out = torch.full((r, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        ops.linear_raw(x[:r], packed, out, gated=mode == "gated")
+        return out
+
+    whole = project(rows[-1])
+    for r in rows[:-1]:
+        assert torch.equal(project(r), whole[:r]), r
+    if mode == "parts":  # the bound of the test of the partials above
+        width = k // whole.shape[1]
+        for i in range(whole.shape[1]):
+            xs, ws = x[:, i * width:(i + 1) * width].float(), w[:, i * width:(i + 1) * width].float()
+            assert ((whole[:, i] - xs @ ws.t()).abs() <= (xs.abs() @ ws.abs().t()) * 2.0 ** -16).all(), i
+        return
+    full, err = x.float() @ w.float().t(), _sum_error(x, w)
+    if mode == "plain":
+        _check_rounded(whole, full, max_mismatch=0.01, extra=err)
+        return
+    gu = full.bfloat16().float()
+    g, u = gu[:, :n], gu[:, n:]
+    act = (g * torch.sigmoid(g)).bfloat16().float()
+    dg, du = _bf16_ulp(g) + err[:, :n], _bf16_ulp(u) + err[:, n:]
+    _check_rounded(whole, act * u, max_mismatch=0.02, extra=1.1 * u.abs() * dg + (act.abs() + dg) * du)
+
+
 @pytest.mark.parametrize("rows,k,n", [(17, 544, 112), (64, 96, 16), (33, 2048, 4096), (65, 2048, 4224),
                                       (129, 2048, 4096), (241, 2048, 4224), (256, 2048, 4096), (65, 5280, 4112),
                                       (113, 5280, 4096), (128, 5280, 4112)])
 def test_streaming_form_at_ring_and_tile_edges(rows: int, k: int, n: int) -> None:
     """The streaming form at 64 contraction steps (whole turns of its weight ring) and 165 (part of a
-    turn and of a chunk), column tiles that do not fill the last workgroup, rows one past a tile,
-    and two shapes beside them on the row kernel, from a strided x and into a strided y: plain and
-    gated."""
+    turn and of a chunk), column tiles that do not fill the last workgroup and rows one past a tile,
+    and beside it two small shapes on the row kernel (544 and 96 wide), from a strided x and into a
+    strided y: plain and gated."""
 
     from continuous_depth_batching_amd import ops
 
