@@ -239,13 +239,13 @@ __global__ void __launch_bounds__(MAXT) linear_kernel(LinearParams p) {
 // that adds them in range order and rounds once (the residual RMSNorm). Wave w
 // owns column tile w; weight blocks stream into a ring of kPartsStages chunks of
 // registers, and x goes through LDS, double-buffered, in operand order. A range
-// is only 16 to 70 steps: the ring holds 16 of them, loaded before anything is
+// is only 16 to 70 steps: the ring holds 16 of them (8 with two-step chunks), loaded before anything is
 // waited for, and the chunk loop unrolls completely, so the launch is close to
 // one memory round trip. The streaming form below, whose first product waits for
 // its producer's first chunk, is slower here (us, cold weights): 5632 -> 2048 at
 // 1 / 16 / 48 / 64 rows 5.7 / 5.8 / 7.4 / 7.8 against 6.4 / 6.6 / 7.7 / 8.4;
 // 2048 -> 2048 at 1 row 3.9 against 4.1; 5280 -> 5280 at 1 / 16 rows 10.8 / 11.2
-// against 11.6 / 12.1. Above those rows it is the faster one (see dispatch_parts).
+// against 11.6 / 12.1. dispatch_parts has the lines above those rows.
 // ---------------------------------------------------------------------------
 constexpr int kPartsStages = 4;
 
@@ -396,12 +396,14 @@ int launch_linear_parts(LinearParams prm, hipStream_t stream) {
 // weight stream never runs ahead of x by more than x's own prefetch. With x in a
 // wave of its own the two run at their own depths. Against the form before it
 // (x loaded and stored to LDS by the waves that multiply; cold weights, us):
-//   2048 -> 6144, 200 rows            15.2 -> 12.9    100 rows  11.1 -> 10.5
-//   2048 -> 2 x 5632 gated, 200 rows  24.0 -> 19.3    100 rows  17.2 -> 14.9
-//   5632 -> 2048, 4 K ranges, 200     13.5 -> 12.0    100 rows  10.5 ->  9.1
-//   5280 -> 2 x 17920 gated, 100      118  -> 70 (5.4 TB/s of weights)
-//   5280 -> 15840, 100 rows           51   -> 40
-//   17920 -> 5280, 4 K ranges, 100    78   -> 42      256 rows   138 -> 60
+//   2048 -> 6144, 200 rows            14.7 -> 12.9    100 rows  10.9 ->  9.5
+//   2048 -> 2 x 5632 gated, 200 rows  22.0 -> 18.4    100 rows  16.5 -> 14.3
+//   5632 -> 2048, 4 K ranges, 200     12.4 -> 11.8
+//   5280 -> 2 x 17920 gated, 100      112  -> 70 (5.4 TB/s of weights)
+//   5280 -> 15840, 100 rows           44   -> 40
+//   17920 -> 5280, 4 K ranges, 100    76   -> 41      256 rows   131 -> 59
+// At 200 rows the gated one takes twice the time of its weight bytes and no resource counted so
+// far is at its limit: a CU pulls some 19 B/clk, its products take 6 us and its LDS reads 5.
 // ---------------------------------------------------------------------------
 constexpr int kStreamSteps = 4;        // SC: contraction steps per x chunk (256 bytes of a row)
 constexpr int kStreamRing = 8;         // RW: weight steps in flight per consumer wave
@@ -782,10 +784,10 @@ int launch_stream_rows(const LinearParams& prm, const StreamTile& t, StreamMode 
 
 // The tile that makes the busiest CU pull the fewest bytes: workgroups are dealt evenly over
 // 256 CUs, so a CU runs ceil(workgroups / 256) of them, and each pulls its rows of x and its
-// columns of W once per contraction step. Against a sweep of every tile over the Ouro-1.4B and
-// Huginn-0125 shapes from 1 to 256 rows the choice is within 4% of the best one (200 rows,
-// 2048 -> 2 x 5632 gated: chosen 112 rows x 3 tile pairs, 236 workgroups, 18.3 us; 112 x 4,
-// 176 workgroups, 19.7; 64 x 3, 472 workgroups, 24).
+// columns of W once per contraction step. Against a sweep of the three to five cheapest tiles at 2 to 12
+// row counts per Ouro-1.4B and Huginn-0125 shape the choice is the best or within 4% of it, but for
+// 2048 -> 6144 at 48 and 224 rows (6 and 8%) and 5280 -> 5280 at 128 rows (6%). 200 rows, 2048 -> 2 x
+// 5632 gated: chosen 112 rows x 3 tile pairs, 236 workgroups, 18.3 us; 112 x 4, 176 workgroups, 19.8.
 StreamTile choose_stream_tile(const LinearParams& prm, StreamMode mode, int splits) {
   const int row_tiles = (prm.M + 15) / 16, col_tiles = prm.N / 16;
   StreamTile best{1, 1, 1};
@@ -887,9 +889,10 @@ int dispatch_parts(const LinearParams& prm, int splits, hipStream_t stream) {
 }
 
 // The row kernel keeps every shape of at most 64 rows that wide_path does not name. The streaming
-// form is faster for some of them (2048 -> 2 x 5632 gated at 16 rows 11.4 -> 10.0 us, 5280 -> 2 x
-// 17920 72 -> 61), but it adds all of K in one accumulator where the row kernel adds four or eight
-// partial sums, and its rounding error against 64 bits must not grow.
+// form is faster for many of them (2048 -> 2 x 5632 gated at 16 rows 11.4 -> 10.0 us; 5280 -> 2 x 17920
+// at 16 / 32 / 64 rows 72 / 81 / 105 -> 61 / 62 / 63 and 5280 -> 15840 at 64 rows 56 -> 33, so that 64
+// rows take longer than 65), but it adds all of K in one accumulator where the row kernel adds four or
+// eight partial sums, and its rounding error against 64 bits must not grow.
 int dispatch_linear(const LinearParams& prm, bool gated, hipStream_t stream) {
   if (wide_path(prm)) return dispatch_stream(prm, gated ? StreamMode::kGated : StreamMode::kPlain, 1, stream);
   if (prm.M <= 16) return dispatch_rows<1, 4>(prm, gated, 8, stream);

@@ -692,7 +692,7 @@ __global__ void __launch_bounds__(kThreads) rope_kv_write_kernel(RopeWriteParams
 
 // The same in 16-byte units, D / C lanes per head. The lanes of a head end anywhere in a wave, so most
 // waves hold query and key heads and rotate both on one path: as two branches they ran one after the
-// other, loads and all (55 heads x 96 in bf16, 4000 tokens 62 -> 58 us, 64 tokens 4.5 -> 4.0; 16 heads
+// other, loads and all (55 heads x 96 in bf16, 4000 tokens 64 -> 61 us, 64 tokens 4.5 -> 3.9; 16 heads
 // x 128 in float, 1000 tokens 15.0 -> 13.8). Where a wave holds one kind the branches cost less, so
 // sixteenths keep them (12 + 4 heads x 64, 64 tokens 2.5 us against 2.7).
 template <typename T, int D>
@@ -773,7 +773,7 @@ int launch_rope_write(void (*kernel)(RopeWriteParams), int64_t groups, const Rop
 // Sixteenths of a head are 8 or 16 bytes for bf16 heads of 64 and 128 and float heads of 64: one
 // access per lane and row part. The other heads (12 bytes, three 4-byte accesses; 24 and 32
 // bytes, several with gaps between the lanes) take 16-byte units where everything is aligned to
-// them: 55 heads x 96 in bf16, 4000 tokens, 70 -> 58 us, 64 tokens 4.3 -> 4.0; 16 heads
+// them: 55 heads x 96 in bf16, 4000 tokens, 71 -> 61 us, 64 tokens 4.4 -> 3.9; 16 heads
 // x 128 in float, 4000 tokens, 54 -> 45 us, 100 tokens 3.6 -> 3.3. (8-byte sixteenths in 16-byte
 // units were slower: 12 + 4 heads x 64, 2000 tokens, 5.0 -> 7.2 us.) Not so in bf16 while the launch is
 // latency and each wave of sixteenths (four heads) is of one kind: 16 + 4 heads, 64 tokens 2.65 us
