@@ -408,7 +408,6 @@ int launch_linear_parts(LinearParams prm, hipStream_t stream) {
 constexpr int kStreamSteps = 4;        // SC: contraction steps per x chunk (256 bytes of a row)
 constexpr int kStreamRing = 8;         // RW: weight steps in flight per consumer wave
 constexpr int kStreamMaxConsumers = 6;
-constexpr int kStreamCus = 256;        // CUs the tile and form choices spread workgroups over
 // S: x stages in LDS. A stage is MT * SC KiB; eight row tiles fit three (and keep the
 // producer's loads in flight under the 63 a wave can count).
 template <int MT> constexpr int kStreamStages = MT < 8 ? 4 : 3;
@@ -755,6 +754,11 @@ int dispatch_rows(const LinearParams& prm, bool gated, int max_waves, hipStream_
                : launch_linear<MT, 1, S, false>(prm, stream, max_waves);
 }
 
+// Workgroups on the fullest XCD of a launch that keeps all row ranges of a (column range, K range)
+// pair on one XCD and deals the pairs over the eight.
+constexpr int kXcdCus = 32;
+int64_t xcd_groups(int64_t pairs, int row_ranges) { return (pairs + 7) / 8 * row_ranges; }
+
 enum class StreamMode { kPlain, kGated, kParts };
 
 struct StreamTile {
@@ -782,8 +786,8 @@ int launch_stream_rows(const LinearParams& prm, const StreamTile& t, StreamMode 
                     : launch_stream<MT, 1, false, true>(prm, t, splits, stream);
 }
 
-// The tile that makes the busiest CU pull the fewest bytes: workgroups are dealt evenly over
-// 256 CUs, so a CU runs ceil(workgroups / 256) of them, and each pulls its rows of x and its
+// The tile that makes the busiest CU pull the fewest bytes: an XCD deals its workgroups evenly over its
+// CUs, so a CU of the fullest one runs ceil(workgroups / 32) of them, and each pulls its rows of x and its
 // columns of W once per contraction step. Against a sweep of the three to five cheapest tiles at 2 to 12
 // row counts per Ouro-1.4B and Huginn-0125 shape the choice is the best or within 4% of it, but for
 // 2048 -> 6144 at 48 and 224 rows (6 and 8%) and 5280 -> 5280 at 128 rows (6%). 200 rows, 2048 -> 2 x
@@ -797,8 +801,9 @@ StreamTile choose_stream_tile(const LinearParams& prm, StreamMode mode, int spli
       for (int c = 2; c <= kStreamMaxConsumers; ++c) {
         const int cols = c * ntw;
         if (ntw == 2 && cols <= kStreamMaxConsumers) continue;  // one tile per wave covers it
-        const int64_t groups = (int64_t)((col_tiles + cols - 1) / cols) * splits * ((row_tiles + mt - 1) / mt);
-        const int64_t cost = (groups + kStreamCus - 1) / kStreamCus * (mt + cols * (mode == StreamMode::kGated ? 2 : 1));
+        const int64_t groups =
+            xcd_groups((int64_t)((col_tiles + cols - 1) / cols) * splits, (row_tiles + mt - 1) / mt);
+        const int64_t cost = (groups + kXcdCus - 1) / kXcdCus * (mt + cols * (mode == StreamMode::kGated ? 2 : 1));
         if (cost <= best_cost) {  // a tie goes to the taller tile: fewer row ranges re-read W from L2
           best_cost = cost;
           best = StreamTile{mt, ntw, c};
@@ -855,22 +860,25 @@ int parts_splits(int64_t rows, int32_t out_features, int32_t in_features) {
 }
 
 // Whether the few-row form with row ranges of 16 * mt rows gives nearly every CU one workgroup and
-// none a second: from `least` workgroups to kStreamCus.
+// none a second: at least `least` workgroups on an XCD's 32 CUs and no more than those.
 bool fills_cus_once(const LinearParams& prm, int splits, int mt, int least) {
-  const int groups = (prm.N / 16 + 3) / 4 * splits * ((prm.M + 16 * mt - 1) / (16 * mt));
-  return groups >= least && groups <= kStreamCus;
+  const int64_t groups =
+      xcd_groups((int64_t)((prm.N / 16 + 3) / 4) * splits, (prm.M + 16 * mt - 1) / (16 * mt));
+  return groups >= least && groups <= kXcdCus;
 }
 
 // The few-row form where it measured faster than the streaming form's chosen tile: up to the row counts
 // of the first lines whatever the width (figures at its kernel), and above where its workgroups fill
 // the CUs once. us, few-row / streaming:
-//   5280 -> 5280, 249 workgroups: 17 rows 11.5 / 12.3, 32 11.9 / 12.7, 48 13.0 / 13.7, 64 14.3 / 14.6
-//   5280 -> 4096 (192) 24 rows 10.5 / 11.0; -> 3584 (168) 10.3 / 10.2; -> 2048 (96) 9.7 / 8.3
-//   2048 -> 2048, 97 and 128 rows (256): 5.5 / 5.5, 5.7 / 5.8; 65 and 96 rows (192) 5.4 / 5.1, 5.65 / 5.35
-//   5632 -> 2048, 65 rows (256): 8.7 / 8.6, 80 8.8 / 9.0, 104 9.0 / 9.2, 128 9.5 / 9.8;
-//   5632 -> 1536 (192) 96 rows 8.5 / 8.1
-// With a second round of workgroups the streaming form is faster: 5280 -> 5280 at 100 rows 23.1 / 17.1,
-// 5632 -> 2048 at 200 rows 13.5 / 12.0, 17920 -> 5280 at 32 / 100 rows 38.6 / 34.1 and 78 / 42.
+//   5280 -> 5280 (32 an XCD): 17 rows 11.5 / 12.3, 32 11.9 / 12.7, 48 13.0 / 13.7, 64 14.3 / 14.6
+//   5280 -> 4096 (24) 24 rows 10.5 / 11.0; -> 3584 (21) 10.3 / 10.2; -> 2048 (12) 9.7 / 8.3, but at 100
+//   rows (24) 10.4 / 11.0; 17920 -> 2048 (32) 40 rows 15.3 / 16.0
+//   2048 -> 2048, 97 and 128 rows (32): 5.5 / 5.5, 5.7 / 5.8; 65 and 96 rows (24) 5.4 / 5.1, 5.65 / 5.35
+//   5632 -> 2048, 65 rows (32): 8.7 / 8.6, 80 8.8 / 9.0, 104 9.0 / 9.2, 128 9.5 / 9.8;
+//   5632 -> 1536 (24) 96 rows 8.5 / 8.1
+// With a second round of workgroups the streaming form is faster: 5280 -> 5280 at 100 rows 25.2 / 19.4,
+// 5632 -> 2048 at 200 rows 12.4 / 11.8, 17920 -> 5280 at 32 / 100 rows 35.8 / 33.5 and 76 / 41; with only
+// one XCD a workgroup over (5280 -> 1792 at 160 rows, 33) 18.1 / 12.0.
 int dispatch_parts(const LinearParams& prm, int splits, hipStream_t stream) {
   if (prm.K == 2048 && prm.M <= 32) return launch_linear_parts<1, 4, 16, 4>(prm, stream);
   if (prm.K == 2048 && prm.M <= 64) return launch_linear_parts<2, 4, 16, 4>(prm, stream);
@@ -879,11 +887,13 @@ int dispatch_parts(const LinearParams& prm, int splits, hipStream_t stream) {
   if (prm.K == 5632 && prm.M <= 64) return launch_linear_parts<2, 4, 44, 4>(prm, stream);
   if (prm.K == 5280 && prm.M <= 16) return launch_linear_parts<1, 4, 55, 3, true>(prm, stream);
   if (prm.K == 17920 && prm.M <= 16) return launch_linear_parts<1, 4, 70, 8, true>(prm, stream);
-  if (prm.K == 5280 && prm.M <= 64 && fills_cus_once(prm, splits, 4, 192))
+  if (prm.K == 5280 && fills_cus_once(prm, splits, 4, 24))
     return launch_linear_parts<4, 2, 55, 3, true>(prm, stream);
-  if (prm.K == 2048 && prm.M <= 128 && fills_cus_once(prm, splits, 2, 196))
+  if (prm.K == 17920 && prm.M <= 64 && fills_cus_once(prm, splits, 4, 25))
+    return launch_linear_parts<4, 2, 70, 8, true>(prm, stream);
+  if (prm.K == 2048 && prm.M <= 128 && fills_cus_once(prm, splits, 2, 25))
     return launch_linear_parts<2, 4, 32, 2>(prm, stream);
-  if (prm.K == 5632 && prm.M <= 128 && fills_cus_once(prm, splits, 4, 196))
+  if (prm.K == 5632 && prm.M <= 128 && fills_cus_once(prm, splits, 4, 25))
     return launch_linear_parts<4, 2, 44, 4>(prm, stream);
   return dispatch_stream(prm, StreamMode::kParts, splits, stream);
 }

@@ -357,15 +357,17 @@ def test_streamed_partials_at_row_range_edges(rows: int, k: int, n: int) -> None
 
 @pytest.mark.parametrize("k,n,rows", [(5280, 5280, (17, 33, 64, 65)), (5280, 4096, (17, 64)), (5280, 4032, (64,)),
                                       (2048, 2048, (65, 96, 97, 128)), (2048, 2560, (65, 96, 97)),
-                                      (5632, 2048, (65, 81, 128, 129)), (5632, 1600, (65, 128))])
+                                      (5632, 2048, (65, 81, 128, 129)), (5632, 1600, (65, 128)),
+                                      (5280, 1280, (65, 129, 193, 224)), (5280, 1792, (160, 192, 224)),
+                                      (5280, 2048, (64, 65, 128)), (17920, 2048, (17, 40)), (17920, 1536, (17, 40))])
 def test_split_k_forms_agree_where_the_shape_changes_them(k: int, n: int, rows: tuple[int, ...]) -> None:
     """Row counts and widths on both sides of the lines between the few-row and the streaming form.
     Both add a K range's steps in order in one accumulator, so a row's partials have the bits of the
-    largest batch with the same ranges (streaming: 256 rows, or 128 for a 2048-wide input)."""
+    largest batch with the same ranges (256 rows, 128 for a 2048-wide input, 64 for a 17920-wide one)."""
 
     from continuous_depth_batching_amd import ops
 
-    most = 128 if k == 2048 else 256
+    most = {2048: 128, 17920: 64}.get(k, 256)
     x, w = _inputs(most, k, n, seed=k + n)
     packed = ops.pack_linear_weight(w)
 
